@@ -324,6 +324,8 @@ __device__ inline double bisect(const double a[4], double lo, double hi)
     if (cubic_at(a, hi) == 0.0) return hi;
     for (int it = 0; it < 80; it++) {
         const double mid = 0.5 * (lo + hi);
+        // neighbours: every further step leaves lo and hi as they are
+        if (mid == lo || mid == hi) break;
         const double pm = cubic_at(a, mid);
         if (pm == 0.0) return mid;
         if ((pm < 0.0) == (plo < 0.0)) {

@@ -9,14 +9,14 @@
 // random_device-seeded engine), so a fixed index set gives one defined
 // inlier count per hypothesis.
 //
-// GPU layout: a 256-thread workgroup owns 256 hypotheses of one pair. Each
-// lane fits one hypothesis in registers (fgeom::fit8) into LDS; then each
-// wavefront scores its 64 hypotheses one at a time, lanes striding over the
-// correspondences staged in LDS tiles of 2048, counting inliers with
-// ballot + popcount on the scalar unit.
+// GPU layout: a workgroup of four wavefronts fits its hypotheses one per lane
+// (fgeom::fit8) into LDS, then counts their inliers over all correspondences
+// with the matrix-core screen of screen.hpp (fundamental matrices) or one lane
+// per hypothesis (homographies).
 #include "internal.hpp"
 #include "fgeom.hpp"
 #include "hgeom.hpp"
+#include "screen.hpp"
 #include <algorithm>
 
 namespace rsfm_amd {
@@ -94,10 +94,10 @@ constexpr int kScoreThreads = 64;
 constexpr int kScoreWaves = RSFM_SCORE_WAVES;
 constexpr int kScoreBlock = kScoreThreads * kScoreWaves;
 
-// points [beg, end) of wavefront w: contiguous parts starting on multiples of 8
-__device__ inline void wave_range(uint32_t n, uint32_t w, uint32_t& beg, uint32_t& end)
+// points [beg, end) of wavefront w of `waves`: contiguous parts starting on multiples of 8
+__device__ inline void wave_range(uint32_t n, uint32_t w, uint32_t waves, uint32_t& beg, uint32_t& end)
 {
-    const uint32_t part = ((n + kScoreWaves - 1) / kScoreWaves + 7u) & ~7u;
+    const uint32_t part = ((n + waves - 1) / waves + 7u) & ~7u;
     beg = min(n, w * part);
     end = min(n, beg + part);
 }
@@ -161,7 +161,7 @@ __global__ __launch_bounds__(kScoreBlock) void score_kernel(const Src batch, flo
     uint32_t cnt = 0;
     if (ok) {
         uint32_t beg, end;
-        wave_range(n, w, beg, end);
+        wave_range(n, w, kScoreWaves, beg, end);
         // the offset is hidden from the uniformity analysis so the loads take
         // the vector memory path (in-order vmcnt, so the prefetch overlaps);
         // all 64 lanes read the same address, one cache line per wavefront
@@ -179,6 +179,108 @@ __global__ __launch_bounds__(kScoreBlock) void score_kernel(const Src batch, flo
     if (T.models) {
 #pragma unroll
         for (int q = 0; q < 9; q++) T.models[(size_t)h * 9 + q] = F[q];
+    }
+}
+
+// Box of the pair's points for the screen, by the calling waves' nThreads
+// threads (t of them): per-wave parts into S.part.
+template <class Sm>
+__device__ inline void box_scan(Sm& S, const float4* __restrict__ P, uint32_t n, uint32_t t, uint32_t nThreads)
+{
+    screen::BoxPart b;
+    screen::box_init(b);
+    uint32_t i = t;
+    for (; i + 3 * nThreads < n; i += 4 * nThreads) {
+        const float4 p0 = P[i], p1 = P[i + nThreads], p2 = P[i + 2 * nThreads], p3 = P[i + 3 * nThreads];
+        screen::box_add(b, p0);
+        screen::box_add(b, p1);
+        screen::box_add(b, p2);
+        screen::box_add(b, p3);
+    }
+    for (; i < n; i += nThreads) screen::box_add(b, P[i]);
+    screen::box_wave_reduce(b);
+    if ((threadIdx.x & 63) == 0) S.part[threadIdx.x >> 6] = b;
+}
+
+// the whole box from the parts of waves [first, kWaves)
+template <class Sm>
+__device__ inline screen::Box box_join(const Sm& S, uint32_t first, uint32_t n)
+{
+    screen::BoxPart b = S.part[first];
+    for (uint32_t w = first + 1; w < Sm::kWaves; w++) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            b.lo[k] = fminf(b.lo[k], S.part[w].lo[k]);
+            b.hi[k] = fmaxf(b.hi[k], S.part[w].hi[k]);
+        }
+        b.odd |= S.part[w].odd;
+    }
+    return screen::box_finish(b, n);
+}
+
+// Scoring of fundamental matrices: a workgroup of eight wavefronts holds 64 kFit
+// hypotheses, fitted one per lane by its first kFit wavefronts while the others
+// scan the pair's box; then the wavefronts count the inliers of 16 kNB
+// hypotheses each, kSplit of them sharing the points, with the matrix-core
+// screen. Coordinates that the screen's bound does not cover (not finite, above
+// 2^20, all equal) take the exact loop.
+
+template <int kMode, int kWaves, int kFit, int kNB, class Src>
+__global__ __launch_bounds__(64 * kWaves, 4) void score_screen_kernel(const Src batch, float t2, float s0, float s1)
+{
+    constexpr uint32_t kHyp = 64 * kFit;
+    constexpr uint32_t kGroups = kHyp / (16 * kNB);       // waves with models of their own
+    constexpr int kSplit = kWaves / kGroups;
+    static_assert(kGroups * kSplit == kWaves && kFit < kWaves, "waves and hypotheses");
+    const Wg3 wg = xcd_local_block();  // all hypothesis blocks of a pair share one L2
+    const DevTask& T = batch[wg.y];
+    if (wg.x * kHyp >= T.H) return;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const uint32_t n = task_n(T);
+    __shared__ screen::Smem<kWaves, 2> S;
+    __shared__ float sF[9][kHyp];
+    __shared__ uint32_t sOk[kHyp], sCnt[kHyp];
+    if (w < kFit) {
+        float F[9];
+        const bool ok = fit_hypothesis<kMode>(T, n, wg.x * kHyp + tid, s0, s1, F);
+#pragma unroll
+        for (int q = 0; q < 9; q++) sF[q][tid] = ok ? F[q] : 0.f;
+        sOk[tid] = ok ? 1u : 0u;
+        sCnt[tid] = 0u;
+    }
+    else box_scan(S, T.pts, n, tid - kHyp, 64 * kWaves - kHyp);
+    __syncthreads();
+    if (n >= (uint32_t)sample_size<kMode>()) {
+        const screen::Box box = box_join(S, kFit, n);
+        auto model = [&](uint32_t k, float F[9]) {
+#pragma unroll
+            for (int q = 0; q < 9; q++) F[q] = sF[q][k];
+            return sOk[k] != 0;
+        };
+        if (!box.odd) {
+            screen::v8h be[kNB], bq[kMode == 1 ? 1 : 2][kNB];
+            float d2[kNB], cc[kNB];
+            const uint32_t base = (w % kGroups) * 16 * kNB;
+            screen::load_models<kMode, kNB>(S, box, base, 16 * kNB, t2, model, be, bq, d2, cc);
+            screen::count_points<kMode, kNB, kSplit>(S, box, T.pts, n, t2, base, w / kGroups, be, bq, d2, cc, sCnt, model);
+        } else {
+            uint32_t beg, end;
+            wave_range(n, w, kWaves, beg, end);
+            for (uint32_t g = 0; g < (uint32_t)kFit; g++) {
+                float F[9];
+                if (!model(g * 64 + lane, F)) continue;
+                const uint32_t c = count_inliers<kMode>(F, T.pts + beg, end - beg, t2);
+                if (c) atomicAdd(&sCnt[g * 64 + lane], c);
+            }
+        }
+    }
+    __syncthreads();
+    const uint32_t h = wg.x * kHyp + tid;
+    if (tid >= kHyp || h >= T.H) return;
+    T.counts[h] = sOk[tid] ? sCnt[tid] : 0u;
+    if (T.models) {
+#pragma unroll
+        for (int q = 0; q < 9; q++) T.models[(size_t)h * 9 + q] = sF[q][tid];
     }
 }
 
@@ -288,58 +390,34 @@ __device__ inline int fit_hypothesis7(const DevTask& T, uint32_t n, uint32_t h, 
 }
 
 // 7-point scoring. A workgroup takes kS7Samples samples, one per lane of its
-// first two wavefronts: every such lane solves its sample (up to three F) and
-// the workgroup's M models are listed in LDS in sample order (a scan of the
-// model counts). Lane l of every wavefront then holds models l, l + 64, ...
-// (R = ceil(M / 64) of them, at most six) in registers and tests each point
-// of its quarter of the correspondences against all R, as score_kernel walks
-// them; the four partial counts are added with LDS atomics. A sample with one
+// first two wavefronts: every such lane solves its sample (up to three F)
+// while the others scan the pair's box, and the workgroup's M models are
+// listed in LDS in sample order (a scan of the model counts). Wavefront w then
+// counts the inliers of models 16 R w .. (R = ceil(M / 128), at most three
+// blocks of 16) over all points with the matrix-core screen. A sample with one
 // real root thus takes one model slot instead of three (about 2.5 models per
-// sample with 8K-keypoint pairs: R = 5 instead of six slots per lane), and
-// every point load feeds R tests. Each sample then reports its best model
-// (most inliers, the first on ties) and that count.
+// sample with 8K-keypoint pairs). Each sample then reports its best model
+// (most inliers, the first on ties) and that count. 32 pairs x 4096 samples x
+// 1400 points on average, two-sided test: 468 -> 288 us against the exact test
+// on every point, of which the solver takes 100.
 constexpr uint32_t kS7Samples = 128;
-constexpr int kS7MaxRounds = (int)(kS7Samples * kMaxF7 / 64);
+constexpr int kS7Waves = 8, kS7Block = 64 * kS7Waves;
 constexpr uint32_t kS7MaxModels = kS7Samples * kMaxF7;
-static_assert(kS7Samples <= kScoreBlock && kS7Samples % 64 == 0, "samples are fitted one per lane");
+static_assert(kS7Samples < kS7Block && kS7Samples % 64 == 0, "samples are fitted one per lane");
 
-// inliers of the lane's R models among P[0, m): the next four points are in
-// flight while the current four are tested (four, not eight: the R models
-// already hold up to 54 registers, and the kernel keeps four waves per SIMD)
-template <int kMode, int R>
-__device__ inline void count7(const float (&F)[kS7MaxRounds][9], const float4* __restrict__ P, uint32_t m, float t2,
-                              uint32_t (&c)[kS7MaxRounds])
+// the wave's 16 R models (base, count of them) over all points
+template <int kMode, int R, class Sm, class Model>
+__device__ inline void count7(Sm& S, const screen::Box& box, const float4* __restrict__ P, uint32_t n, float t2,
+                              uint32_t base, uint32_t count, uint32_t* cnt, Model model)
 {
-    auto test = [&](const float4& p) {
-#pragma unroll
-        for (int r = 0; r < R; r++) c[r] += fgeom::inlier<kMode>(F[r], p, t2) ? 1u : 0u;
-    };
-    uint32_t i = 0;
-    if (m >= 4) {
-        float4 q0 = P[0], q1 = P[1], q2 = P[2], q3 = P[3];
-        for (; i + 8 <= m; i += 4) {
-            const float4* __restrict__ Q = P + i + 4;
-            const float4 n0 = Q[0], n1 = Q[1], n2 = Q[2], n3 = Q[3];
-            test(q0);
-            test(q1);
-            test(q2);
-            test(q3);
-            q0 = n0;
-            q1 = n1;
-            q2 = n2;
-            q3 = n3;
-        }
-        test(q0);
-        test(q1);
-        test(q2);
-        test(q3);
-        i += 4;
-    }
-    for (; i < m; i++) test(P[i]);
+    screen::v8h be[R], bq[kMode == 1 ? 1 : 2][R];
+    float d2[R], cc[R];
+    screen::load_models<kMode, R>(S, box, base, count, t2, model, be, bq, d2, cc);
+    screen::count_points<kMode, R, 1>(S, box, P, n, t2, base, 0, be, bq, d2, cc, cnt, model);
 }
 
 template <int kMode, class Src>
-__global__ __launch_bounds__(kScoreBlock) void score7_kernel(const Src batch, float t2, float s0, float s1)
+__global__ __launch_bounds__(kS7Block, 4) void score7_kernel(const Src batch, float t2, float s0, float s1)
 {
     const Wg3 wg = xcd_local_block();
     const DevTask& T = batch[wg.y];
@@ -347,12 +425,14 @@ __global__ __launch_bounds__(kScoreBlock) void score7_kernel(const Src batch, fl
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const uint32_t h = wg.x * kS7Samples + tid;
     const uint32_t n = task_n(T);
+    __shared__ screen::Smem<kS7Waves, 1> S;  // two workgroups per CU
     __shared__ float sF[9][kS7MaxModels];
     __shared__ uint32_t sCnt[kS7MaxModels];
     __shared__ uint32_t sWaveModels[kS7Samples / 64];
-    for (uint32_t k = tid; k < kS7MaxModels; k += kScoreBlock) sCnt[k] = 0u;
+    for (uint32_t k = tid; k < kS7MaxModels; k += kS7Block) sCnt[k] = 0u;
     float Fw[kMaxF7][9];  // written by the solver with a running index
     const int nm = tid < kS7Samples ? fit_hypothesis7(T, n, h, s0, s1, Fw) : 0;
+    if (tid >= kS7Samples) box_scan(S, T.pts, n, tid - kS7Samples, kS7Block - kS7Samples);
     // the models' place in the list: prefix of nm in lane order (the lanes
     // past the samples add nothing)
     uint32_t inc = (uint32_t)nm;
@@ -375,36 +455,31 @@ __global__ __launch_bounds__(kScoreBlock) void score7_kernel(const Src batch, fl
     uint32_t M = 0;
 #pragma unroll
     for (uint32_t k = 0; k < kS7Samples / 64; k++) M += sWaveModels[k];
-    const int R = (int)((M + 63) / 64);
-    float F[kS7MaxRounds][9];  // model r * 64 + lane; zero (never an inlier) past the list
+    const uint32_t R = (M + 16 * (uint32_t)kS7Waves - 1) / (16 * (uint32_t)kS7Waves);
+    if (R > 0) {
+        const screen::Box box = box_join(S, kS7Samples / 64, n);
+        auto model = [&](uint32_t k, float F[9]) {
 #pragma unroll
-    for (int r = 0; r < kS7MaxRounds; r++) {
-        const uint32_t k = (uint32_t)r * 64 + lane;
-#pragma unroll
-        for (int q = 0; q < 9; q++) F[r][q] = k < M ? sF[q][k] : 0.f;
-    }
-    uint32_t c[kS7MaxRounds] = {0u, 0u, 0u, 0u, 0u, 0u};
-    uint32_t beg, end;
-    wave_range(n, w, beg, end);
-    // the offset is hidden from the uniformity analysis so the loads take the
-    // vector memory path (see score_kernel)
-    uint32_t base = beg;
-    asm volatile("" : "+v"(base));
-    const float4* P = T.pts + base;
-    const uint32_t m = end - beg;
-    switch (R) {
-        case 1: count7<kMode, 1>(F, P, m, t2, c); break;
-        case 2: count7<kMode, 2>(F, P, m, t2, c); break;
-        case 3: count7<kMode, 3>(F, P, m, t2, c); break;
-        case 4: count7<kMode, 4>(F, P, m, t2, c); break;
-        case 5: count7<kMode, 5>(F, P, m, t2, c); break;
-        case 6: count7<kMode, 6>(F, P, m, t2, c); break;
-        default: break;
-    }
-#pragma unroll
-    for (int r = 0; r < kS7MaxRounds; r++) {
-        const uint32_t k = (uint32_t)r * 64 + lane;
-        if (r < R && k < M) atomicAdd(&sCnt[k], c[r]);
+            for (int q = 0; q < 9; q++) F[q] = sF[q][k];
+            return true;
+        };
+        if (!box.odd) {
+            const uint32_t base = w * 16 * R, count = M > base ? min(M - base, 16 * R) : 0u;
+            switch (R) {
+                case 1: count7<kMode, 1>(S, box, T.pts, n, t2, base, count, sCnt, model); break;
+                case 2: count7<kMode, 2>(S, box, T.pts, n, t2, base, count, sCnt, model); break;
+                default: count7<kMode, 3>(S, box, T.pts, n, t2, base, count, sCnt, model); break;
+            }
+        } else {
+            uint32_t beg, end;
+            wave_range(n, w, (uint32_t)kS7Waves, beg, end);
+            for (uint32_t k = lane; k < M; k += 64) {
+                float F[9];
+                model(k, F);
+                const uint32_t c = count_inliers<kMode>(F, T.pts + beg, end - beg, t2);
+                if (c) atomicAdd(&sCnt[k], c);
+            }
+        }
     }
     __syncthreads();
     if (tid >= kS7Samples || h >= T.H) return;
@@ -690,6 +765,34 @@ int launch_sample_table(const SampleTask* tasks, uint32_t nTasks, uint32_t maxH,
     return check_launch("sample table");
 }
 
+// Scores of nTasks tasks of at most maxH hypotheses; kind = model kind. A
+// 256-hypothesis workgroup stages each point for four times the models of a
+// 64-hypothesis one, which in turn keeps more workgroups in flight: at 12
+// pairs x 4096 hypotheses x 1300-2400 points (192 or 768 workgroups) the wide
+// form takes 53 us and the narrow one 58 us, at one pair (16 or 64) only the
+// narrow one spreads the fits. 32 pairs x 4096 x 2454 points: 208 -> 98 us
+// against one exact test per lane and trip (VALU issue 84% busy; 46.6 M vector
+// instructions instead of 110 M), 64 pairs of the affine-filtered batch 218 ->
+// 139 us.
+constexpr uint32_t kWideMin = 128;
+template <class Src>
+static int launch_score(const Src& src, uint32_t nTasks, uint32_t maxH, float t2, int kind, float s0, float s1,
+                        hipStream_t stream, const char* name)
+{
+    if (kind == 2) {
+        score_kernel<2><<<dim3(div_up(maxH, kScoreThreads), nTasks), kScoreBlock, 0, stream>>>(src, t2, s0, s1);
+    } else if (div_up(maxH, 256) * nTasks >= kWideMin) {
+        const dim3 grid(div_up(maxH, 256), nTasks);
+        if (kind == 0) score_screen_kernel<0, 8, 4, 2><<<grid, 512, 0, stream>>>(src, t2, s0, s1);
+        else score_screen_kernel<1, 8, 4, 4><<<grid, 512, 0, stream>>>(src, t2, s0, s1);
+    } else {
+        const dim3 grid(div_up(maxH, 64), nTasks);
+        if (kind == 0) score_screen_kernel<0, 4, 1, 1><<<grid, 256, 0, stream>>>(src, t2, s0, s1);
+        else score_screen_kernel<1, 4, 1, 1><<<grid, 256, 0, stream>>>(src, t2, s0, s1);
+    }
+    return check_launch(name);
+}
+
 int launch_score_table(const DevTask* tasks, uint32_t nTasks, uint32_t maxH, float threshold, int mode,
                        float minSepSq0, float minSepSq1, hipStream_t stream, bool withBest)
 {
@@ -697,12 +800,7 @@ int launch_score_table(const DevTask* tasks, uint32_t nTasks, uint32_t maxH, flo
     if (nTasks == 0) return RSFM_OK;
     const float t2 = threshold * threshold;
     const InTable<DevTask> src{tasks};
-    if (maxH > 0) {
-        const dim3 grid(div_up(maxH, kScoreThreads), nTasks);
-        if (mode == 0) score_kernel<0><<<grid, kScoreBlock, 0, stream>>>(src, t2, minSepSq0, minSepSq1);
-        else score_kernel<1><<<grid, kScoreBlock, 0, stream>>>(src, t2, minSepSq0, minSepSq1);
-        RSFM_CHECK(check_launch("ransac score table"));
-    }
+    if (maxH > 0) RSFM_CHECK(launch_score(src, nTasks, maxH, t2, mode, minSepSq0, minSepSq1, stream, "ransac score table"));
     if (!withBest) return RSFM_OK;
     if (mode == 0) best_kernel<0><<<nTasks, kBestThreads, 0, stream>>>(src, t2, minSepSq0, minSepSq1);
     else best_kernel<1><<<nTasks, kBestThreads, 0, stream>>>(src, t2, minSepSq0, minSepSq1);
@@ -718,8 +816,8 @@ int launch_score7_table(const DevTask* tasks, uint32_t nTasks, uint32_t maxH, fl
     const InTable<DevTask> src{tasks};
     if (maxH > 0) {
         const dim3 grid(div_up(maxH, kS7Samples), nTasks);
-        if (mode == 0) score7_kernel<0><<<grid, kScoreBlock, 0, stream>>>(src, t2, minSepSq0, minSepSq1);
-        else score7_kernel<1><<<grid, kScoreBlock, 0, stream>>>(src, t2, minSepSq0, minSepSq1);
+        if (mode == 0) score7_kernel<0><<<grid, kS7Block, 0, stream>>>(src, t2, minSepSq0, minSepSq1);
+        else score7_kernel<1><<<grid, kS7Block, 0, stream>>>(src, t2, minSepSq0, minSepSq1);
         RSFM_CHECK(check_launch("ransac7 score table"));
     }
     if (mode == 0) best7_kernel<0><<<nTasks, kThreads, 0, stream>>>(src, t2, minSepSq0, minSepSq1);
@@ -757,13 +855,7 @@ static int run_hypotheses(const rsfm_ransac_task* tasks, size_t nbTasks, float t
                                  t.counts, t.models, t.best, t.inlierMask};
             maxH = std::max(maxH, t.nbHyp);
         }
-        if (maxH > 0) {
-            const dim3 grid(div_up(maxH, kScoreThreads), (uint32_t)n);
-            if (kind == 0) score_kernel<0><<<grid, kScoreBlock, 0, stream>>>(batch, t2, minSepSq0, minSepSq1);
-            else if (kind == 1) score_kernel<1><<<grid, kScoreBlock, 0, stream>>>(batch, t2, minSepSq0, minSepSq1);
-            else score_kernel<2><<<grid, kScoreBlock, 0, stream>>>(batch, t2, minSepSq0, minSepSq1);
-            RSFM_CHECK(check_launch(name));
-        }
+        if (maxH > 0) RSFM_CHECK(launch_score(batch, (uint32_t)n, maxH, t2, kind, minSepSq0, minSepSq1, stream, name));
         bool anyBest = false;
         for (size_t i = 0; i < n; i++) anyBest |= batch.t[i].best != nullptr || batch.t[i].mask != nullptr;
         if (anyBest) {
@@ -888,8 +980,8 @@ extern "C" int rsfm_ransac_f7(const rsfm_ransac_task* tasks, size_t nbTasks, flo
         }
         if (maxH > 0) {
             const dim3 grid(div_up(maxH, kS7Samples), (uint32_t)n);
-            if (mode == 0) score7_kernel<0><<<grid, kScoreBlock, 0, stream>>>(batch, t2, minSepSq0, minSepSq1);
-            else score7_kernel<1><<<grid, kScoreBlock, 0, stream>>>(batch, t2, minSepSq0, minSepSq1);
+            if (mode == 0) score7_kernel<0><<<grid, kS7Block, 0, stream>>>(batch, t2, minSepSq0, minSepSq1);
+            else score7_kernel<1><<<grid, kS7Block, 0, stream>>>(batch, t2, minSepSq0, minSepSq1);
             RSFM_CHECK(check_launch("ransac7 score"));
         }
         bool anyBest = false;
