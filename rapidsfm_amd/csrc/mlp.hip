@@ -29,6 +29,7 @@ namespace rsfm_amd {
 namespace mlp {
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int kH = 64;
@@ -119,14 +120,17 @@ __device__ inline v16f bias_block(const Ops& S, int L, int b, int hi)
 }
 
 // ReLU of two output blocks, packed as the four B operands of the next layer
+// (NaN to 0). One v_med3 per unit: of x > 0 ? x : 0 the compiler makes two
+// v_max, the first to quiet NaNs, and of a med3 with known bounds as well.
 __device__ inline void relu_pack(const v16f (&a)[2], v8bf (&B)[4])
 {
+    float zero = 0.f, inf = __builtin_inff();
+    asm("" : "+s"(zero), "+s"(inf));
 #pragma unroll
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            const float x = a[t >> 1][8 * (t & 1) + j];
-            B[t][j] = to_bf(x > 0.f ? x : 0.f);
+            B[t][j] = to_bf(__builtin_amdgcn_fmed3f(a[t >> 1][8 * (t & 1) + j], zero, inf));
         }
 }
 
@@ -187,18 +191,134 @@ __device__ inline float forward_tile(const Ops& S, const float* __restrict__ X, 
     return z + S.b4;
 }
 
-__global__ __launch_bounds__(256) void forward_kernel(const float* __restrict__ P, const float* __restrict__ X,
-                                                      uint32_t n, float* __restrict__ prob)
+// Forward pass alone. Every operand stays in registers over the wave's tiles
+// (18 weight operands, the hidden biases as accumulator starts, the output
+// weights as bf16 pairs: about 220 VGPRs, two waves per SIMD), so a tile costs
+// no LDS traffic; reading the weights and biases from LDS for every tile (42
+// reads of 16 B) set the time before: 1 M matches 58 -> 25 us. Layer 1 has 8 of
+// its 16 K slots free, three of which carry the bias split into three bf16
+// parts (24 bits) against ones. ReLU and packing are 1.5 instructions per unit,
+// the output layer 16 v_dot2 per match.
+struct FwdOps {
+    v8bf w1[2][64];
+    v8bf w2[2][4][64];
+    v8bf w3[2][4][64];
+    float bias[2][2][2][16];  // layers 2, 3: [layer][block][hi][v] in output-block order
+    v2bf w4[2][16];           // [hi][8 t + j / 2]
+    float b4;
+};
+
+__device__ void build_fwd(FwdOps& S, const float* __restrict__ P)
 {
-    __shared__ Ops S;
-    build_ops(S, P);
+    const int tid = threadIdx.x;
+    for (int e = tid; e < 2 * 64; e += blockDim.x) {
+        const int rb = e >> 6, lane = e & 63, o = 32 * rb + (lane & 31);
+        v8bf r;
+#pragma unroll
+        for (int j = 0; j < 8; j++) r[j] = to_bf(P[OFF_W1 + o * 8 + j]);
+        if (lane >= 32) {
+            float b = P[OFF_B1 + o];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                r[j] = to_bf(j < 3 ? b : 0.f);
+                b = isfinite(from_bf(r[j])) ? b - from_bf(r[j]) : 0.f;
+            }
+        }
+        S.w1[rb][lane] = r;
+    }
+    for (int e = tid; e < 2 * 4 * 64; e += blockDim.x) {
+        const int rb = e >> 8, t = (e >> 6) & 3, lane = e & 63, m = lane & 31, hi = lane >> 5;
+        v8bf a2, a3;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int u = 16 * t + sigma(8 * hi + j), r = 32 * rb + m;
+            a2[j] = to_bf(P[OFF_W2 + r * kH + u]);
+            a3[j] = to_bf(P[OFF_W3 + r * kH + u]);
+        }
+        S.w2[rb][t][lane] = a2;
+        S.w3[rb][t][lane] = a3;
+    }
+    for (int e = tid; e < 2 * 2 * 2 * 16; e += blockDim.x) {
+        const int L = e >> 6, b = (e >> 5) & 1, hi = (e >> 4) & 1, v = e & 15;
+        S.bias[L][b][hi][v] = P[(L == 0 ? OFF_B2 : OFF_B3) + 32 * b + 8 * (v >> 2) + 4 * hi + (v & 3)];
+    }
+    for (int e = tid; e < 64; e += blockDim.x) {
+        const int hi = e >> 5, bv = e & 31, b = bv >> 4, v = bv & 15;
+        S.w4[hi][bv >> 1][bv & 1] = to_bf(P[OFF_W4 + 32 * b + 8 * (v >> 2) + 4 * hi + (v & 3)]);
+    }
+    if (tid == 0) S.b4 = P[OFF_B4];
+}
+
+__global__ __launch_bounds__(256, 2) void forward_kernel(const float* __restrict__ P, const float* __restrict__ X,
+                                                         uint32_t n, float* __restrict__ prob)
+{
+    __shared__ FwdOps S;
+    build_fwd(S, P);
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (uint32_t base = (blockIdx.x * kWaves + wave) * 32u; base < n; base += gridDim.x * kWaves * 32u) {
-        Acts A;
-        const float z = forward_tile(S, X, n, base, lane, A);
-        const uint32_t idx = base + lane;
-        if (lane < 32 && idx < n) prob[idx] = 1.f / (1.f + __expf(-z));
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hi = lane >> 5;
+    v8bf w1[2], w2[2][4], w3[2][4];
+    v16f b2[2], b3[2];
+    v2bf w4[16];
+#pragma unroll
+    for (int rb = 0; rb < 2; rb++) {
+        w1[rb] = S.w1[rb][lane];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            w2[rb][t] = S.w2[rb][t][lane];
+            w3[rb][t] = S.w3[rb][t][lane];
+        }
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            b2[rb][v] = S.bias[0][rb][hi][v];
+            b3[rb][v] = S.bias[1][rb][hi][v];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 16; k++) w4[k] = S.w4[hi][k];
+    const float b4 = S.b4;
+    const uint32_t step = gridDim.x * kWaves * 32u;
+    uint32_t base = (blockIdx.x * kWaves + wave) * 32u;
+    // the lower half-wave's lanes load one match each, the upper half stages ones
+    float4 p = make_float4(1.f, 1.f, 1.f, 0.f), q = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto fetch = [&](uint32_t at) {
+        if (hi == 0 && at < n) {
+            p = *reinterpret_cast<const float4*>(X + (size_t)at * 8);
+            q = *reinterpret_cast<const float4*>(X + (size_t)at * 8 + 4);
+        }
+    };
+    fetch(base + lane);
+    for (; base < n; base += step) {
+        const v8bf x = {to_bf(p.x), to_bf(p.y), to_bf(p.z), to_bf(p.w), to_bf(q.x), to_bf(q.y), to_bf(q.z), to_bf(q.w)};
+        if (base + step < n) fetch(base + step + lane);
+        v16f a[2], c[2];
+        v8bf h[4];
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) a[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w1[rb], x, zero16(), 0, 0, 0);
+        relu_pack(a, h);
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) c[rb] = b2[rb];
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int rb = 0; rb < 2; rb++) c[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w2[rb][t], h[t], c[rb], 0, 0, 0);
+        relu_pack(c, h);
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) a[rb] = b3[rb];
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int rb = 0; rb < 2; rb++) a[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w3[rb][t], h[t], a[rb], 0, 0, 0);
+        relu_pack(a, h);
+        float z0 = 0.f, z1 = 0.f;
+#pragma unroll
+        for (int k = 0; k < 16; k += 2) {
+            z0 = __builtin_amdgcn_fdot2_f32_bf16(w4[k], v2bf{h[k >> 2][2 * (k & 3)], h[k >> 2][2 * (k & 3) + 1]}, z0, false);
+            z1 = __builtin_amdgcn_fdot2_f32_bf16(w4[k + 1], v2bf{h[k >> 2][2 * (k & 3) + 2], h[k >> 2][2 * (k & 3) + 3]}, z1, false);
+        }
+        float z = z0 + z1;
+        z += __shfl_xor(z, 32);
+        z += b4;
+        if (hi == 0 && base + lane < n) prob[base + lane] = 1.f / (1.f + __expf(-z));
     }
 }
 
@@ -407,14 +527,37 @@ __global__ __launch_bounds__(256) void grad_kernel(const float* __restrict__ P, 
     }
 }
 
-// grad[p] = sum over partials in workgroup order (deterministic); loss = mean
-__global__ void reduce_kernel(const float* __restrict__ partials, uint32_t nPart, uint32_t n, float* __restrict__ grad,
-                              float* __restrict__ loss)
+// grad[p] = sum over the partials in a fixed order (deterministic): eight
+// thread groups of a workgroup take every eighth partial each, eight loads in
+// flight, and their sums are added in group order; loss = mean. One thread per
+// parameter, all partials in turn, left 36 workgroups waiting for one load at a
+// time: 64 partials 16.2 -> 4 us.
+constexpr int kRedParams = 32, kRedGroups = 8;
+__global__ __launch_bounds__(kRedParams * kRedGroups) void reduce_kernel(const float* __restrict__ partials, uint32_t nPart,
+                                                                         uint32_t n, float* __restrict__ grad,
+                                                                         float* __restrict__ loss)
 {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p > (uint32_t)kNParam) return;
+    __shared__ float sum[kRedGroups][kRedParams];
+    const uint32_t c = threadIdx.x % kRedParams, g = threadIdx.x / kRedParams;
+    const uint32_t p = blockIdx.x * kRedParams + c;
+    const bool live = p <= (uint32_t)kNParam;
+    const float* src = partials + (live ? p : 0u);
     float s = 0.f;
-    for (uint32_t w = 0; w < nPart; w++) s += partials[(size_t)w * (kNParam + 1) + p];
+    uint32_t w = g;
+    for (; w + 7 * kRedGroups < nPart; w += 8 * kRedGroups) {
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = src[(size_t)(w + k * kRedGroups) * (kNParam + 1)];
+#pragma unroll
+        for (int k = 0; k < 8; k++) s += v[k];
+    }
+    for (; w < nPart; w += kRedGroups) s += src[(size_t)w * (kNParam + 1)];
+    sum[g][c] = s;
+    __syncthreads();
+    if (g != 0 || !live) return;
+    s = 0.f;
+#pragma unroll
+    for (int k = 0; k < kRedGroups; k++) s += sum[k][c];
     if (p < (uint32_t)kNParam)
         grad[p] = s;
     else if (loss)
@@ -502,7 +645,7 @@ extern "C" int rsfm_mlp_forward(const float* params, const float* x, uint32_t n,
     RSFM_RETURN_IF(n > 0 && (x == nullptr || prob == nullptr), RSFM_ERR_INVALID, "mlp forward: x/prob null");
     RSFM_RETURN_IF(reinterpret_cast<uintptr_t>(x) % 16 != 0, RSFM_ERR_INVALID, "mlp forward: x must be 16-byte aligned");
     if (n == 0) return RSFM_OK;
-    const uint32_t grid = std::min<uint32_t>(1024u, div_up(n, mlp::kWaves * 32));
+    const uint32_t grid = std::min<uint32_t>(512u, div_up(n, mlp::kWaves * 32));
     mlp::forward_kernel<<<grid, 256, 0, stream>>>(params, x, n, prob);
     return check_launch("mlp forward");
 }
@@ -529,7 +672,7 @@ extern "C" int rsfm_mlp_grad(const float* params, const float* x, const float* y
     float* part = static_cast<float*>(workspace);
     mlp::grad_kernel<<<grid, 256, 0, stream>>>(params, x, y, n, 1.f / (float)n, part);
     RSFM_CHECK(check_launch("mlp grad"));
-    mlp::reduce_kernel<<<div_up(mlp::kNParam + 1, 256), 256, 0, stream>>>(part, grid, n, grad, loss);
+    mlp::reduce_kernel<<<div_up(mlp::kNParam + 1, mlp::kRedParams), mlp::kRedParams * mlp::kRedGroups, 0, stream>>>(part, grid, n, grad, loss);
     return check_launch("mlp grad reduce");
 }
 
