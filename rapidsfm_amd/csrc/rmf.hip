@@ -16,6 +16,7 @@
 #include "internal.hpp"
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace rsfm_amd {
@@ -24,39 +25,35 @@ namespace rmf {
 constexpr int kCta = 128;
 constexpr uint32_t kMinInliers = 6;
 
+// a cell's 3 x 3 neighbourhood: its matches are three runs of the cell-ordered
+// array, one per cell row (cells of a row are consecutive)
 struct Cells {
-    uint32_t start[9], size[9], sum;
+    uint32_t start[3], end[3];  // end: of the runs' concatenation
+    uint32_t sum;
 };
 
 __device__ inline void cells_init(Cells& c, const uint32_t* bounds, uint32_t cols, uint32_t rows, uint32_t bx, uint32_t by)
 {
     c.sum = 0;
+    const uint32_t n0 = bx > 0 ? bx - 1 : 0, n1 = min(bx + 1, cols - 1);
 #pragma unroll
-    for (int t = 0; t < 9; t++) {
-        const int m = (int)by - 1 + t / 3, n = (int)bx - 1 + t % 3;
-        if (m >= 0 && m < (int)rows && n >= 0 && n < (int)cols) {
-            const uint32_t idx = (uint32_t)m * cols + (uint32_t)n;
-            c.start[t] = bounds[idx];
-            c.size[t] = bounds[idx + 1] - bounds[idx];
-        } else {
-            c.start[t] = 0;
-            c.size[t] = 0;
+    for (int t = 0; t < 3; t++) {
+        const int m = (int)by - 1 + t;
+        c.start[t] = 0;
+        if (m >= 0 && m < (int)rows) {
+            c.start[t] = bounds[(uint32_t)m * cols + n0];
+            c.sum += bounds[(uint32_t)m * cols + n1 + 1] - c.start[t];
         }
-        c.sum += c.size[t];
+        c.end[t] = c.sum;
     }
 }
 
+// place of the neighbourhood's idx-th match (idx < sum)
 __device__ inline uint32_t cells_map(const Cells& c, uint32_t idx)
 {
-    uint32_t acc = 0;
-#pragma unroll
-    for (int i = 0; i < 9; i++) {
-        if (c.size[i] == 0) continue;
-        const uint32_t nxt = acc + c.size[i];
-        if (idx < nxt) return c.start[i] + (idx - acc);
-        acc = nxt;
-    }
-    return ~0u;
+    if (idx < c.end[0]) return c.start[0] + idx;
+    if (idx < c.end[1]) return c.start[1] + (idx - c.end[0]);
+    return c.start[2] + (idx - c.end[1]);
 }
 
 __device__ inline float sq_threshold(const float T[6], float threshold)
@@ -75,13 +72,305 @@ __device__ inline bool is_inlier(const float T[6], float4 p, float sq)
     return d0 * d0 + d1 * d1 < sq;
 }
 
-__device__ inline uint32_t count_inliers(const Cells& c, const float T[6], const float4* m, float threshold)
+// Inlier counts of one affine per lane over a neighbourhood, by the matrix
+// cores. d0 = T0 x + T1 y + T2 - x' and d1 are matrix products with f16 halves
+// (22 bits) of the coordinates about the neighbourhood's first match and of the
+// coefficients, ten of K = 16 slots each; s = d0^2 + d1^2 - sq then differs from
+// the FP32 test's by at most the model's c (below), so s < -c and s > c have
+// the exact outcome and only tests between are done by is_inlier. Four vector
+// instructions per test instead of seventeen: v_fma twice, v_alignbit (sign
+// bits, one popcount per 32 tests) and, per four tests, the least |s| less c
+// (v_min3, v_min, v_sub, v_alignbit).
+// 64 pairs of about 4000 matches in 16 x 12 cells, 256 hypotheses: best affine
+// 327 -> 126 us, votes 284 -> 110 us (the exact test per lane and match had 17
+// instructions and its match's load in the chain).
+// The bound, u = 2^-24, M = the largest magnitudes in the neighbourhood about
+// its first match, m the same in pixels: a staged term is off by 13 u (the
+// subtraction, two splits of 2^-22, the dropped lo * lo), the matrix unit's
+// FP32 sum by 10 u of the terms' magnitudes (5.4 u measured), halves below
+// f16's normal range by 2^-14 absolute; the exact expression rounds at most
+// 3 u (|T0| mx + |T1| my) + 2 u (|T2| + mx').
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+constexpr uint32_t kTiles = 16, kChunk = kTiles * 16;  // matches staged at a time
+constexpr float kScale = 64.f;                         // coefficients are staged times 2^6
+constexpr float kFar = 32768.f;
+
+struct Half2 {
+    _Float16 h, l;
+};
+__device__ inline Half2 split(float x)
 {
+    asm("" : "+v"(x));  // one rounding for both uses of x (no v_fma_mixlo_f16)
+    Half2 r;
+    r.h = (_Float16)x;
+    r.l = (_Float16)(x - (float)r.h);
+    return r;
+}
+
+struct CountSmem {
+    v4h tile[kTiles][64];             // matches as matrix operands, [lane] = (match, K group)
+    float4 raw[kChunk];               // the same matches as they are
+    v4h model[kCta / 64][2][2][64];   // [wave][d0, d1][K group][model]
+    float T[kCta / 64][6][64];
+    float sq[kCta / 64][64];
+    float big[kCta / 64][4];
+};
+
+// a neighbourhood's centre (its first match) and largest magnitudes about it
+struct Frame {
+    float cx, cy, cz, cw, x, y, z, w;
+    bool odd;  // coordinates beyond the bound: every test is exact
+};
+
+__device__ inline float wave_max(float x)
+{
+    const auto dpp = [](float v, auto k) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(k)::value, 0xF, 0xF, true));
+    };
+    x = fmaxf(x, dpp(x, std::integral_constant<int, 0xB1>{}));   // quad_perm: neighbour
+    x = fmaxf(x, dpp(x, std::integral_constant<int, 0x4E>{}));   // quad_perm: other pair
+    x = fmaxf(x, dpp(x, std::integral_constant<int, 0x141>{}));  // row_half_mirror
+    x = fmaxf(x, dpp(x, std::integral_constant<int, 0x140>{}));  // row_mirror
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+__device__ inline void frame_add(Frame& f, const float4& p)
+{
+    f.x = fmaxf(f.x, fabsf(p.x - f.cx));
+    f.y = fmaxf(f.y, fabsf(p.y - f.cy));
+    f.z = fmaxf(f.z, fabsf(p.z - f.cz));
+    f.w = fmaxf(f.w, fabsf(p.w - f.cw));
+    f.odd = f.odd || !(fabsf(p.x) + fabsf(p.y) + fabsf(p.z) + fabsf(p.w) < 1e6f);
+}
+
+// match i of the chunk (valid: there is one) to S.tile: K groups
+// {x.h x.h x.l 64}, {y.h y.h y.l 64}, {x'.h x'.l y'.h y'.l}, {pad, 1024, 0, 0}
+__device__ __forceinline__ void stage_match(CountSmem& S, const Frame& f, uint32_t i, bool valid, const float4& p)
+{
+    const _Float16 z = (_Float16)0.f;
+    const Half2 x = split(p.x - f.cx), y = split(p.y - f.cy), u = split(p.z - f.cz), v = split(p.w - f.cw);
+    v4h* t = S.tile[i >> 4] + (i & 15);
+    t[0] = valid ? v4h{x.h, x.h, x.l, (_Float16)kScale} : v4h{z, z, z, z};
+    t[16] = valid ? v4h{y.h, y.h, y.l, (_Float16)kScale} : v4h{z, z, z, z};
+    t[32] = valid ? v4h{u.h, u.l, v.h, v.l} : v4h{z, z, z, z};
+    t[48] = valid ? v4h{z, (_Float16)1024.f, z, z} : v4h{(_Float16)kFar, z, z, z};
+}
+
+// The neighbourhood's frame and, when it fits one chunk, its matches staged
+// (each is loaded once). All threads of the workgroup call it; c.sum > 0.
+__device__ __forceinline__ Frame stage_cell(CountSmem& S, const Cells& c, const float4* __restrict__ m)
+{
+    constexpr uint32_t kPer = kChunk / kCta;
+    const uint32_t tid = threadIdx.x;
+    const bool one = c.sum <= kChunk;
+    float4 p[kPer];
+    if (one) {
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; u++) p[u] = m[cells_map(c, min(tid + u * kCta, c.sum - 1))];
+    }
+    const float4 o = m[cells_map(c, 0)];
+    Frame f{o.x, o.y, o.z, o.w, 0.f, 0.f, 0.f, 0.f, false};
+    if (one) {
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; u++) frame_add(f, p[u]);
+    } else {
+        for (uint32_t k = tid; k < c.sum; k += kCta) frame_add(f, m[cells_map(c, k)]);
+    }
+    f.x = wave_max(f.odd ? 1e6f : f.x);
+    f.y = wave_max(f.y);
+    f.z = wave_max(f.z);
+    f.w = wave_max(f.w);
+    if ((tid & 63) == 0) {
+        S.big[tid >> 6][0] = f.x;
+        S.big[tid >> 6][1] = f.y;
+        S.big[tid >> 6][2] = f.z;
+        S.big[tid >> 6][3] = f.w;
+    }
+    if (one) {
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; u++) {
+            const uint32_t i = tid + u * kCta;
+            if (i < ((c.sum + 15) & ~15u)) {
+                stage_match(S, f, i, i < c.sum, p[u]);
+                S.raw[i] = p[u];
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kCta / 64; w++) {
+        f.x = fmaxf(f.x, S.big[w][0]);
+        f.y = fmaxf(f.y, S.big[w][1]);
+        f.z = fmaxf(f.z, S.big[w][2]);
+        f.w = fmaxf(f.w, S.big[w][3]);
+    }
+    f.odd = !(fmaxf(fmaxf(f.x, f.y), fmaxf(f.z, f.w)) < 30000.f);
+    return f;
+}
+
+// matches [at, at + kChunk) of a longer neighbourhood
+__device__ __forceinline__ void stage_chunk(CountSmem& S, const Cells& c, const Frame& f, const float4* __restrict__ m, uint32_t at)
+{
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < kChunk; i += kCta) {
+        const float4 p = m[cells_map(c, min(at + i, c.sum - 1))];
+        stage_match(S, f, i, at + i < c.sum, p);
+        S.raw[i] = p;
+    }
+    __syncthreads();
+}
+
+// inliers of the lane's affine T (live: it has any) over the neighbourhood;
+// every thread of the workgroup calls it
+__device__ __forceinline__ uint32_t count_inliers(CountSmem& S, const Cells& c, const Frame& f, const float T[6], bool live,
+                                         const float4* __restrict__ m, float threshold)
+{
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, q = lane >> 4;
     const float sq = sq_threshold(T, threshold);
-    uint32_t cnt = 0;
-    for (int i = 0; i < 9; i++)
-        for (uint32_t k = c.start[i]; k < c.start[i] + c.size[i]; k++) cnt += is_inlier(T, m[k], sq);
-    return cnt;
+    live = live && sq > 0.f;  // false for NaN too: such a model has no inliers
+    if (f.odd) {
+        uint32_t cnt = 0;
+        if (live)
+            for (uint32_t k = 0; k < c.sum; k++) cnt += is_inlier(T, m[cells_map(c, k)], sq);
+        return cnt;
+    }
+    // the model about the frame's centre, its operands and c
+    const float t0 = fabsf(T[0]), t1 = fabsf(T[1]), t3 = fabsf(T[3]), t4 = fabsf(T[4]);
+    const double o0 = (double)T[0] * f.cx + (double)T[1] * f.cy + ((double)T[2] - f.cz);
+    const double o1 = (double)T[3] * f.cx + (double)T[4] * f.cy + ((double)T[5] - f.cw);
+    const float a0 = (float)fabs(o0), a1 = (float)fabs(o1);
+    const float px = f.x + fabsf(f.cx), py = f.y + fabsf(f.cy), pz = f.z + fabsf(f.cz), pw = f.w + fabsf(f.cw);
+    const float u = 5.9604645e-8f;
+    // an inlier's x' is within the threshold of the model's value: larger ones do not reach the boundary
+    const float th = sqrtf(sq);
+    const float z0 = t0 * f.x + t1 * f.y + a0, z1 = t3 * f.x + t4 * f.y + a1;
+    const float e0 = u * (23.f * (z0 + fminf(f.z, z0 + 2.f * th)) + 3.f * (t0 * px + t1 * py) + 2.f * (fabsf(T[2]) + pz)) +
+                     6.2e-5f * (t0 + t1 + 3.f) + 1e-6f * (f.x + f.y);
+    const float e1 = u * (23.f * (z1 + fminf(f.w, z1 + 2.f * th)) + 3.f * (t3 * px + t4 * py) + 2.f * (fabsf(T[5]) + pw)) +
+                     6.2e-5f * (t3 + t4 + 3.f) + 1e-6f * (f.x + f.y);
+    const float cc = 1.05f * (2.f * th * (e0 + e1) + e0 * e0 + e1 * e1 + 16.f * u * sq);
+    // a model that maps the whole neighbourhood further from its matches than the
+    // threshold (another cell's, extrapolated) has no inlier; the margins cover e0, e1
+    if (a0 * 0.9999f > t0 * f.x + t1 * f.y + f.z + 2.f * th || a1 * 0.9999f > t3 * f.x + t4 * f.y + f.w + 2.f * th) live = false;
+    // beyond f16's range: every test of the model is open
+    const bool open = live && !(fmaxf(fmaxf(t0, t1), fmaxf(t3, t4)) < 500.f && fmaxf(a0, a1) < 30000.f && sq < 1e8f && cc < 1e8f);
+    const bool use = live && !open;
+    {
+        const float k = use ? kScale : 0.f, k1 = use ? 1.f : 0.f;
+        const Half2 x0 = split(T[0] * k), y0 = split(T[1] * k), x1 = split(T[3] * k), y1 = split(T[4] * k);
+        const Half2 w0 = split((float)o0 * k1), w1 = split((float)o1 * k1);
+        S.model[wave][0][0][lane] = use ? v4h{x0.h, x0.l, x0.h, w0.h} : v4h{0, 0, 0, 0};
+        S.model[wave][0][1][lane] = use ? v4h{y0.h, y0.l, y0.h, w0.l} : v4h{0, 0, 0, 0};
+        S.model[wave][1][0][lane] = use ? v4h{x1.h, x1.l, x1.h, w1.h} : v4h{0, 0, 0, 0};
+        S.model[wave][1][1][lane] = use ? v4h{y1.h, y1.l, y1.h, w1.l} : v4h{0, 0, 0, 0};
+#pragma unroll
+        for (int k6 = 0; k6 < 6; k6++) S.T[wave][k6][lane] = T[k6];
+        S.sq[wave][lane] = sq;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // operands of the wave's four blocks of 16 models; -sq and c in units of
+    // (64 px)^2. A dead model's third group makes d0 huge; an open one has
+    // s = 0, c = 1.
+    v4h m0[4], m1[4];
+    float sqn[4], cs[4];
+    const _Float16 z = (_Float16)0.f, one = (_Float16)-kScale;
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+        const int src = b * 16 + (int)c16;
+        const float bs = __shfl(use ? sq * (kScale * kScale) : 0.f, src);
+        const float bc = __shfl(use ? cc * (kScale * kScale) : (open ? 1.f : 0.f), src);
+        const bool dead = __shfl(live ? 0 : 1, src) != 0, any = __shfl(use ? 1 : 0, src) != 0;
+        sqn[b] = -bs;
+        cs[b] = bc;
+        if (q < 2) {
+            m0[b] = S.model[wave][0][q][src];
+            m1[b] = S.model[wave][1][q][src];
+        } else if (q == 2) {
+            m0[b] = any ? v4h{one, one, z, z} : v4h{z, z, z, z};
+            m1[b] = any ? v4h{z, z, one, one} : v4h{z, z, z, z};
+        } else {
+            m0[b] = v4h{(_Float16)kFar, dead ? (_Float16)kFar : z, z, z};
+            m1[b] = v4h{z, z, z, z};
+        }
+    }
+    uint32_t acc[4] = {0, 0, 0, 0};
+    for (uint32_t at = 0; at < c.sum; at += kChunk) {
+        if (c.sum > kChunk) stage_chunk(S, c, f, m, at);
+        const uint32_t tiles = min(kTiles, (c.sum - at + 15) / 16);
+        for (uint32_t g0 = 0; g0 < tiles; g0 += 8) {
+            const uint32_t nt = min(8u, tiles - g0);
+            uint32_t in[4] = {0, 0, 0, 0}, near[4] = {0, 0, 0, 0};
+            for (uint32_t t = 0; t < nt; t++) {
+                const v4h a = S.tile[g0 + t][lane];
+                const v4f zero = {0.f, 0.f, 0.f, 0.f};
+                v4f d0[4], d1[4];
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    d0[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(a, m0[b], zero, 0, 0, 0);
+                    d1[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(a, m1[b], zero, 0, 0, 0);
+                }
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    float s[4];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        s[j] = fmaf(d1[b][j], d1[b][j], fmaf(d0[b][j], d0[b][j], sqn[b]));
+                        in[b] = __builtin_amdgcn_alignbit(in[b], __float_as_uint(s[j]), 31);
+                    }
+                    const float low = fminf(fminf(fminf(fabsf(s[0]), fabsf(s[1])), fabsf(s[2])), fabsf(s[3])) - cs[b];
+                    near[b] = __builtin_amdgcn_alignbit(near[b], __float_as_uint(low), 31);
+                }
+            }
+            // open groups of four tests, each by its lane, exactly
+            while (__any((near[0] | near[1] | near[2] | near[3]) != 0)) {
+                uint32_t w = 0, k = 0;
+#pragma unroll
+                for (int b = 3; b >= 0; b--)
+                    if (near[b]) {
+                        w = near[b];
+                        k = b;
+                    }
+                if (w) {
+                    const uint32_t bit = (uint32_t)__ffs((int)w) - 1u, src = k * 16 + c16;
+                    float M[6];
+#pragma unroll
+                    for (int k6 = 0; k6 < 6; k6++) M[k6] = S.T[wave][k6][src];
+                    const float ms = S.sq[wave][src];
+                    const uint32_t i = (g0 + nt - 1 - bit) * 16 + 4 * q;
+                    uint32_t a = 0;
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; j++)
+                        a += at + i + j < c.sum && is_inlier(M, S.raw[i + j], ms) ? 1u : 0u;
+#pragma unroll
+                    for (int b = 0; b < 4; b++)
+                        if ((uint32_t)b == k) {
+                            near[b] &= w - 1;
+                            in[b] &= ~(15u << (4 * bit));
+                            acc[b] += a;
+                        }
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < 4; b++) acc[b] += (uint32_t)__popc(in[b]);
+        }
+    }
+    // sums over the lane groups; the lane's model is number lane % 16 of block lane / 16
+    uint32_t mine = 0;
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+        uint32_t a = acc[b];
+        a += (uint32_t)__shfl_xor((int)a, 16);
+        a += (uint32_t)__shfl_xor((int)a, 32);
+        if (q == (uint32_t)b) mine = a;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    return live ? mine : 0u;
 }
 
 // solveGaussElim semantics (SfmUtils.hpp:156-184): no pivoting, 3x3 with two right-hand sides
@@ -123,32 +412,41 @@ __device__ inline uint32_t lcg(uint32_t& s)
 }
 
 struct Reducer {
-    uint32_t cnt[kCta / 2];
-    float aff[kCta / 2][6];
+    uint32_t key[kCta / 64];
+    float aff[6];
 };
 
-// CtaReducer::findMax: thread t keeps its value unless t + mid holds a strictly larger count
-__device__ inline void cta_find_max(Reducer& R, uint32_t& cnt, float T[6])
+// CtaReducer::findMax: the largest count; among equals its tree (thread t keeps
+// its value unless t + mid holds a strictly larger count, mid = 64 .. 1) leaves
+// the thread whose reversed index is lowest. The winner's count and affine are
+// returned to every thread.
+__device__ __forceinline__ void cta_find_max(Reducer& R, uint32_t& cnt, float T[6])
 {
-    const uint32_t tid = threadIdx.x;
-    for (uint32_t mid = kCta / 2; mid != 0; mid /= 2) {
-        if (tid >= mid && tid < 2 * mid) {
-            R.cnt[tid - mid] = cnt;
+    static_assert(kCta == 128, "seven index bits");
+    const uint32_t order = 127u - (__brev(threadIdx.x) >> 25);
+    const uint32_t mine = (cnt << 7) | order;  // fewer than 2^25 matches in a neighbourhood
+    uint32_t key = mine;
 #pragma unroll
-            for (int q = 0; q < 6; q++) R.aff[tid - mid][q] = T[q];
-        }
-        __syncthreads();
-        if (tid < mid && cnt < R.cnt[tid]) {
-            cnt = R.cnt[tid];
+    for (int s = 32; s > 0; s >>= 1) key = max(key, (uint32_t)__shfl_xor((int)key, s));
+    if ((threadIdx.x & 63) == 0) R.key[threadIdx.x >> 6] = key;
+    __syncthreads();
+    key = max(R.key[0], R.key[1]);
+    if (mine == key)
 #pragma unroll
-            for (int q = 0; q < 6; q++) T[q] = R.aff[tid][q];
-        }
-        __syncthreads();
-    }
+        for (int q = 0; q < 6; q++) R.aff[q] = T[q];
+    __syncthreads();
+    cnt = key >> 7;
+#pragma unroll
+    for (int q = 0; q < 6; q++) T[q] = R.aff[q];
 }
 
+struct CellSmem {
+    Reducer R;
+    CountSmem C;
+};
+
 // one cell (bx, by): the best of nbTests affine hypotheses
-__device__ inline void best_affine_cell(Reducer& R, float* __restrict__ affine, const float4* __restrict__ m,
+__device__ __forceinline__ void best_affine_cell(CellSmem& S, float* __restrict__ affine, const float4* __restrict__ m,
                                         const uint32_t* __restrict__ bounds, uint32_t cols, uint32_t rows,
                                         uint32_t nbTests, float threshold, uint32_t seed, uint32_t bx, uint32_t by)
 {
@@ -159,53 +457,62 @@ __device__ inline void best_affine_cell(Reducer& R, float* __restrict__ affine, 
         if (threadIdx.x < 6) affine[rank * 6 + threadIdx.x] = __builtin_nanf("");
         return;
     }
+    const Frame f = stage_cell(S.C, c, m);
     float best[6] = {1.f, 0.f, 0.f, 0.f, 1.f, 0.f};
     uint32_t bestCnt = 0;
     uint32_t st = seed + (kCta * rank + threadIdx.x) * 22695477u;
-    for (uint32_t h = threadIdx.x; h < nbTests; h += kCta) {
-        uint32_t idx[3];
-        uint32_t got = 0;
-        while (got < 3) {
-            const uint32_t v = lcg(st) % c.sum;
-            bool dup = false;
-            for (uint32_t q = 0; q < got; q++) dup |= idx[q] == v;
-            if (!dup) idx[got++] = v;
-        }
-        float Ab[3][5];
+    for (uint32_t h0 = 0; h0 < nbTests; h0 += kCta) {
+        bool live = h0 + threadIdx.x < nbTests;
+        float T[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (live) {
+            uint32_t idx[3];
+            uint32_t got = 0;
+            while (got < 3) {
+                const uint32_t v = lcg(st) % c.sum;
+                bool dup = false;
+                for (uint32_t q = 0; q < got; q++) dup |= idx[q] == v;
+                if (!dup) idx[got++] = v;
+            }
+            float Ab[3][5];
 #pragma unroll
-        for (int r = 0; r < 3; r++) {
-            const float4 p = m[cells_map(c, idx[r])];
-            Ab[r][0] = p.x;
-            Ab[r][1] = p.y;
-            Ab[r][2] = 1.f;
-            Ab[r][3] = p.z;
-            Ab[r][4] = p.w;
+            for (int r = 0; r < 3; r++) {
+                const float4 p = c.sum <= kChunk ? S.C.raw[idx[r]] : m[cells_map(c, idx[r])];
+                Ab[r][0] = p.x;
+                Ab[r][1] = p.y;
+                Ab[r][2] = 1.f;
+                Ab[r][3] = p.z;
+                Ab[r][4] = p.w;
+            }
+            float X[3][2];
+            solve_gauss3(Ab, X);
+#pragma unroll
+            for (int r = 0; r < 3; r++) {
+                T[r] = X[r][0];
+                T[3 + r] = X[r][1];
+            }
+            const float sqrScale = T[0] * T[4] - T[1] * T[3];
+            if (sqrScale < 0.0625f || sqrScale > 16.f || !isfinite(sqrScale)) live = false;
         }
-        float X[3][2];
-        solve_gauss3(Ab, X);
-        const float T[6] = {X[0][0], X[1][0], X[2][0], X[0][1], X[1][1], X[2][1]};
-        const float sqrScale = T[0] * T[4] - T[1] * T[3];
-        if (sqrScale < 0.0625f || sqrScale > 16.f || !isfinite(sqrScale)) continue;
-        const uint32_t k = count_inliers(c, T, m, threshold);
+        const uint32_t k = count_inliers(S.C, c, f, T, live, m, threshold);
         if (k > bestCnt) {
             bestCnt = k;
 #pragma unroll
             for (int q = 0; q < 6; q++) best[q] = T[q];
         }
     }
-    cta_find_max(R, bestCnt, best);
+    cta_find_max(S.R, bestCnt, best);
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int q = 0; q < 6; q++) affine[rank * 6 + q] = best[q];
     }
 }
 
-__global__ __launch_bounds__(kCta) void best_affine_kernel(float* __restrict__ affine, const float4* __restrict__ m,
+__global__ __launch_bounds__(kCta, 4) void best_affine_kernel(float* __restrict__ affine, const float4* __restrict__ m,
                                                            const uint32_t* __restrict__ bounds, uint32_t cols,
                                                            uint32_t rows, uint32_t nbTests, float threshold, uint32_t seed)
 {
-    __shared__ Reducer R;
-    best_affine_cell(R, affine, m, bounds, cols, rows, nbTests, threshold, seed, blockIdx.x, blockIdx.y);
+    __shared__ CellSmem S;
+    best_affine_cell(S, affine, m, bounds, cols, rows, nbTests, threshold, seed, blockIdx.x, blockIdx.y);
 }
 
 __device__ inline void vote(uint32_t* votesWords, uint32_t idx)
@@ -213,64 +520,49 @@ __device__ inline void vote(uint32_t* votesWords, uint32_t idx)
     atomicAdd(votesWords + (idx >> 2), 1u << (8 * (idx & 3)));
 }
 
-struct VoteSmem {
-    Reducer R;
-    float best[6];
-    uint32_t bestCnt;
-};
-
 // one cell: its own affine (or, with tryOther, the best of every cell's affine
 // on its neighbourhood) votes for its inliers when it explains >= 6 of them
-__device__ inline void vote_cell(VoteSmem& S, uint32_t* __restrict__ votesWords, const float* __restrict__ affine,
+__device__ __forceinline__ void vote_cell(CellSmem& S, uint32_t* __restrict__ votesWords, const float* __restrict__ affine,
                                  const float4* __restrict__ m, const uint32_t* __restrict__ bounds, uint32_t cols,
                                  uint32_t rows, float threshold, bool tryOther, uint32_t bx, uint32_t by)
 {
     Cells c;
     cells_init(c, bounds, cols, rows, bx, by);
+    if (c.sum < kMinInliers) return;  // nobody can explain that many
     const uint32_t rank = by * cols + bx;
-    const uint32_t nCells = cols * rows;
+    const uint32_t nCells = tryOther ? cols * rows : 1u;
+    const Frame f = stage_cell(S.C, c, m);
     float best[6];
 #pragma unroll
     for (int q = 0; q < 6; q++) best[q] = affine[rank * 6 + q];
     uint32_t bestCnt = 0;
-    if (tryOther) {
-        for (uint32_t n = threadIdx.x; n < nCells; n += kCta) {
-            float T[6];
+    for (uint32_t n0 = 0; n0 < nCells; n0 += kCta) {
+        const uint32_t n = n0 + threadIdx.x;
+        const bool live = n < nCells;
+        float T[6];
 #pragma unroll
-            for (int q = 0; q < 6; q++) T[q] = affine[n * 6 + q];
-            const uint32_t k = count_inliers(c, T, m, threshold);
-            if (k > bestCnt) {
-                bestCnt = k;
+        for (int q = 0; q < 6; q++) T[q] = affine[(tryOther && live ? n : rank) * 6 + q];
+        const uint32_t k = count_inliers(S.C, c, f, T, live, m, threshold);
+        if (k > bestCnt) {
+            bestCnt = k;
 #pragma unroll
-                for (int q = 0; q < 6; q++) best[q] = T[q];
-            }
+            for (int q = 0; q < 6; q++) best[q] = T[q];
         }
-        cta_find_max(S.R, bestCnt, best);
-    } else if (threadIdx.x == 0) {
-        bestCnt = count_inliers(c, best, m, threshold);
     }
-    if (threadIdx.x == 0) {
-        S.bestCnt = bestCnt;
-#pragma unroll
-        for (int q = 0; q < 6; q++) S.best[q] = best[q];
-    }
-    __syncthreads();
-    if (S.bestCnt < kMinInliers) return;
-    float T[6];
-#pragma unroll
-    for (int q = 0; q < 6; q++) T[q] = S.best[q];
-    const float sq = sq_threshold(T, threshold);
+    cta_find_max(S.R, bestCnt, best);
+    if (bestCnt < kMinInliers) return;
+    const float sq = sq_threshold(best, threshold);
     for (uint32_t k = threadIdx.x; k < c.sum; k += kCta) {
         const uint32_t mi = cells_map(c, k);
-        if (is_inlier(T, m[mi], sq)) vote(votesWords, mi);
+        if (is_inlier(best, c.sum <= kChunk ? S.C.raw[k] : m[mi], sq)) vote(votesWords, mi);
     }
 }
 
-__global__ __launch_bounds__(kCta) void vote_kernel(uint32_t* __restrict__ votesWords, const float* __restrict__ affine,
+__global__ __launch_bounds__(kCta, 4) void vote_kernel(uint32_t* __restrict__ votesWords, const float* __restrict__ affine,
                                                     const float4* __restrict__ m, const uint32_t* __restrict__ bounds,
                                                     uint32_t cols, uint32_t rows, float threshold, bool tryOther)
 {
-    __shared__ VoteSmem S;
+    __shared__ CellSmem S;
     vote_cell(S, votesWords, affine, m, bounds, cols, rows, threshold, tryOther, blockIdx.x, blockIdx.y);
 }
 
@@ -300,14 +592,16 @@ struct BinSmem {
     uint32_t cnt[kMaxCells];
     uint32_t cursor[kMaxCells];
     uint16_t waveCnt[kBinWaves][kMaxCells];
-    uint32_t scan[kBinThreads];
+    uint32_t scan[kBinWaves];
 };
 
 // one workgroup per task: votes cleared, cell counts, bounds (exclusive
 // prefix, cells in row-major order), then a stable scatter: points in index
 // order, a point's slot = its cell's start + earlier points of the same cell
-// (ballot peer groups inside a wave, per-wave cell counts across the waves of a
-// round of 1024 points, a running cursor across rounds)
+// (peer groups from ballots inside a wave, per-wave cell counts across the waves of a
+// round of 1024 points, a running cursor across rounds); 64 tasks of about 4000
+// points 39 -> 19 us with peer groups by the cell number's bits and the cell
+// prefix by wave scans
 template <class Src>
 __global__ __launch_bounds__(kBinThreads) void bin_kernel(const Src batch)
 {
@@ -326,16 +620,17 @@ __global__ __launch_bounds__(kBinThreads) void bin_kernel(const Src batch)
     __syncthreads();
     // exclusive prefix over the cells (nCells <= kMaxCells = kBinThreads)
     const uint32_t v = tid < nCells ? S.cnt[tid] : 0u;
-    S.scan[tid] = v;
-    __syncthreads();
-    for (uint32_t off = 1; off < kBinThreads; off <<= 1) {
-        const uint32_t a = tid >= off ? S.scan[tid - off] : 0u;
-        __syncthreads();
-        S.scan[tid] += a;
-        __syncthreads();
+    uint32_t inc = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)inc, o);
+        if (lane >= (uint32_t)o) inc += y;
     }
+    if (lane == 63) S.scan[wave] = inc;
+    __syncthreads();
+    for (uint32_t w = 0; w < wave; w++) inc += S.scan[w];
     if (tid < nCells) {
-        const uint32_t start = S.scan[tid] - v;
+        const uint32_t start = inc - v;
         S.cursor[tid] = start;
         T.bounds[tid] = start;
     }
@@ -351,15 +646,13 @@ __global__ __launch_bounds__(kBinThreads) void bin_kernel(const Src batch)
             cell = cell_of(p.x, p.y, T);
         }
         for (uint32_t c = lane; c < nCells; c += 64) S.waveCnt[wave][c] = 0;
-        // lanes of this wave with the same cell
-        uint64_t peers = 0;
-        uint64_t todo = __ballot(valid);
-        while (todo) {
-            const int leader = __ffsll((unsigned long long)todo) - 1;
-            const uint32_t lc = (uint32_t)__shfl((int)cell, leader);
-            const uint64_t same = __ballot(valid && cell == lc);
-            if (valid && cell == lc) peers = same;
-            todo &= ~same;
+        // lanes of this wave with the same cell: those that agree on every bit of
+        // its number (one ballot a bit; one per distinct cell took up to 64)
+        uint64_t peers = __ballot(valid);
+        for (uint32_t k = 0; (1u << k) < nCells; k++) {
+            const bool bit = (cell >> k) & 1u;
+            const uint64_t set = __ballot(bit);
+            peers &= bit ? set : ~set;
         }
         const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
         const uint32_t rank = (uint32_t)__popcll(peers & below);
@@ -383,19 +676,19 @@ __global__ __launch_bounds__(kBinThreads) void bin_kernel(const Src batch)
 }
 
 template <class Src>
-__global__ __launch_bounds__(kCta) void best_affine_batch_kernel(const Src batch, BatchParams prm)
+__global__ __launch_bounds__(kCta, 4) void best_affine_batch_kernel(const Src batch, BatchParams prm)
 {
-    __shared__ Reducer R;
+    __shared__ CellSmem S;
     const BatchTask& T = batch[blockIdx.z];
     if (blockIdx.x >= T.cols || blockIdx.y >= T.rows || task_n(T) < 16) return;
-    best_affine_cell(R, T.affine, T.reordered, T.bounds, T.cols, T.rows, prm.nbTests, T.threshold, T.seed, blockIdx.x,
+    best_affine_cell(S, T.affine, T.reordered, T.bounds, T.cols, T.rows, prm.nbTests, T.threshold, T.seed, blockIdx.x,
                      blockIdx.y);
 }
 
 template <class Src>
-__global__ __launch_bounds__(kCta) void vote_batch_kernel(const Src batch, BatchParams prm)
+__global__ __launch_bounds__(kCta, 4) void vote_batch_kernel(const Src batch, BatchParams prm)
 {
-    __shared__ VoteSmem S;
+    __shared__ CellSmem S;
     const BatchTask& T = batch[blockIdx.z];
     if (blockIdx.x >= T.cols || blockIdx.y >= T.rows || task_n(T) < 16) return;
     vote_cell(S, reinterpret_cast<uint32_t*>(T.votes), T.affine, T.reordered, T.bounds, T.cols, T.rows, T.threshold,
