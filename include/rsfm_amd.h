@@ -108,7 +108,7 @@ int rsfm_bf_match_u4(const rsfm_bf_task* tasks, size_t nbTasks, hipStream_t stre
 /* top-2 query side + top-1 train side (new). Needs a workspace of
  * rsfm_bf_match_top2_workspace_size() bytes, 256-B aligned: the staging form
  * of each task's train descriptors (132 B per descriptor, nbDescB rounded up
- * to 64), written by the call, and the segment partials of long train sets. */
+ * to 64), written by the call. */
 int rsfm_bf_match_top2_workspace_size(const rsfm_bf_top2_task* tasks, size_t nbTasks, size_t* bytes);
 int rsfm_bf_match_top2(const rsfm_bf_top2_task* tasks, size_t nbTasks, void* workspace,
                        size_t workspaceBytes, hipStream_t stream);
@@ -545,7 +545,7 @@ int rsfm_ransac_sample_indices_batch_k(const rsfm_sample_task* tasks, size_t nbT
  * ImagePair.cpp:148-204). Many pairs of uneven size are matched (top-2 query
  * side, top-1 train side), filtered (ratio test + cross-check + keypoint
  * gather), sampled and scored by one HIP graph launch. All buffers are the
- * caller's except the pipeline's own task tables and partials. Inputs must be
+ * caller's except the pipeline's own task tables and staging. Inputs must be
  * complete when rsfm_pipeline_create is called: it times candidate matcher
  * tilings on them (autotuning) on a private stream before capturing the graph.
  * Results are the same as the individual entry points' (rsfm_bf_match_top2,
@@ -634,7 +634,7 @@ typedef struct rsfm_pipeline_config {
 #define RSFM_PIPELINE_SOLVER_DEGENSAC 1u
 typedef struct rsfm_pipeline_tuning_entry {
     uint32_t segCols, wgPerXcd;
-    float matchMs;             /* fill + match + merge, best of three */
+    float matchMs;             /* preparation + match, best of three */
 } rsfm_pipeline_tuning_entry;
 typedef struct rsfm_pipeline_info_t {
     uint32_t segCols, wgPerXcd, nbTiles;
@@ -644,7 +644,7 @@ typedef struct rsfm_pipeline rsfm_pipeline;
 int rsfm_pipeline_create(const rsfm_pipeline_pair* pairs, size_t nbPairs, const rsfm_pipeline_config* cfg,
                          rsfm_pipeline** out);
 /* one run in flight at a time: the graph's stages share the pipeline's task tables and
- * partials; rsfm_pipeline_destroy waits for the last run's stream */
+ * staging; rsfm_pipeline_destroy waits for the last run's stream */
 int rsfm_pipeline_run(rsfm_pipeline* pipeline, hipStream_t stream);
 int rsfm_pipeline_info(const rsfm_pipeline* pipeline, rsfm_pipeline_info_t* info, rsfm_pipeline_tuning_entry* entries,
                        size_t maxEntries, size_t* nbEntries);

@@ -29,12 +29,13 @@
 //    by atomicMin; at the end of the tile every column within 1 of that
 //    minimum is recomputed exactly on MFMA and merged by a 64-bit atomicMin.
 //  * Segments split the train range when one launch has too few row blocks
-//    to fill 256 CUs; row results then merge by 64-bit atomicMin (top-1) or
-//    through a small workspace and a merge kernel (top-2).
+//    to fill 256 CUs; row results then merge by 64-bit atomicMin, the second
+//    best from the key that loses.
 #include "internal.hpp"
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace rsfm_amd {
@@ -416,10 +417,14 @@ __device__ __forceinline__ void match_tile_top2(const DevTask& T, uint32_t rowBa
                 if (T.nSeg == 1) {
                     T.bestA[row] = k1;
                     T.secondA[row] = k2;
-                } else {
-                    uint64_t* pp = T.part + ((size_t)seg * T.nA + row) * 2;
-                    pp[0] = k1;
-                    pp[1] = k2;
+                } else if (k1 != kNoMatch) {
+                    // several segments, merged in place: of the segment's best and
+                    // the one found there the smaller stays, the other may be the
+                    // second; every key but the smallest reaches secondA once
+                    const uint64_t old = atomicMin(reinterpret_cast<unsigned long long*>(T.bestA + row), (unsigned long long)k1);
+                    const uint64_t c = umin64(umax64(old, k1), k2);
+                    if (c != kNoMatch)
+                        atomicMin(reinterpret_cast<unsigned long long*>(T.secondA + row), (unsigned long long)c);
                 }
             } else if (T.nSeg == 1) {
                 T.bestA[row] = k1;
@@ -529,21 +534,22 @@ __device__ __forceinline__ void match_tile_top2(const DevTask& T, uint32_t rowBa
 // __launch_bounds__(512, 4): 512 threads, at least four waves per SIMD, i.e.
 // at most 128 VGPRs, so two workgroups fit a CU.
 // Top-1 (rsfm_bf_match_u8 / _u4, 8- or 4-bit descriptors).
-template <int kBits>
-__global__ __launch_bounds__(512, 4) void match_top1_kernel(const TaskBatch batch)
+template <int kBits, class Src>
+__global__ __launch_bounds__(512, 4) void match_top1_kernel(const Src batch)
 {
     const Wg3 wg = xcd_local_block();
-    const DevTask& T = batch.t[wg.z];
+    const DevTask& T = batch[wg.z];
     const uint32_t rowBase = wg.x * kBM;
     const uint32_t colBeg = wg.y * T.segCols;
     if (rowBase >= T.nA || colBeg >= T.nB) return;
     match_tile_top2<kBits, false>(T, rowBase, colBeg, wg.y);
 }
 
-__global__ __launch_bounds__(512, 4) void match_top2_kernel(const TaskBatch batch)
+template <class Src>
+__global__ __launch_bounds__(512, 4) void match_top2_kernel(const Src batch)
 {
     const Wg3 wg = xcd_local_block();
-    const DevTask& T = batch.t[wg.z];
+    const DevTask& T = batch[wg.z];
     const uint32_t rowBase = wg.x * kBM;
     const uint32_t colBeg = wg.y * T.segCols;
     if (rowBase >= T.nA || colBeg >= T.nB) return;
@@ -588,24 +594,18 @@ __global__ __launch_bounds__(512, 4) void match_tile_grid_kernel(const DevTask* 
 // each (4-bit descriptors widened to bytes); a workgroup of 256 covers 32
 // columns and the padded column count is a multiple of 64, so a workgroup is
 // wholly inside or outside it. The same threads also set results to "no
-// match": kInitNone leaves them (the pipeline clears its own), kInitTop2 sets
-// the train-side results (merged by atomicMin) and, for a task without train
-// descriptors, the query-side ones (no tile writes them), kInitTop1 sets the
-// train-side and all query-side results (several segments merge them by
-// atomicMin).
-enum : int { kInitNone = 0, kInitTop2 = 1, kInitTop1 = 2 };
+// match": the train side (merged by atomicMin), and the query side where
+// several segments merge it or no tile writes it (no train descriptors).
 template <int kBits, class Src>
-__global__ __launch_bounds__(256) void prep_train_kernel(const Src batch, int init)
+__global__ __launch_bounds__(256) void prep_train_kernel(const Src batch)
 {
     const DevTask& T = batch[blockIdx.z];
     const uint32_t nPad = (T.nB + kBN - 1) / kBN * kBN;
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (init != kInitNone) {
-        if (T.bestB != nullptr && t < T.nB) T.bestB[t] = kNoMatch;
-        if ((T.nB == 0 || init == kInitTop1) && t < T.nA) {
-            T.bestA[t] = kNoMatch;
-            if (T.secondA != nullptr) T.secondA[t] = kNoMatch;
-        }
+    if (T.bestB != nullptr && t < T.nB) T.bestB[t] = kNoMatch;
+    if ((T.nB == 0 || T.nSeg > 1) && t < T.nA) {
+        T.bestA[t] = kNoMatch;
+        if (T.secondA != nullptr) T.secondA[t] = kNoMatch;
     }
     const uint32_t col = t >> 3, sp = t & 7;
     if (T.W == nullptr || col >= nPad) return;
@@ -651,33 +651,17 @@ void place_prep(DevTask& t, uint8_t* ws)
     t.colMin = reinterpret_cast<int32_t*>(ws);
 }
 
-int launch_prep_table(const DevTask* tasks, uint32_t nTasks, uint32_t maxB, hipStream_t stream)
+// threads of one task's preparation: eight per padded train column, one per result
+static uint32_t prep_blocks(uint32_t maxA, uint32_t maxB)
 {
-    if (nTasks == 0 || maxB == 0) return RSFM_OK;
-    const uint32_t nPad = div_up(maxB, (uint32_t)kBN) * kBN;
-    prep_train_kernel<8><<<dim3(nPad * 8 / 256, 1, nTasks), 256, 0, stream>>>(TaskTable{tasks}, kInitNone);
-    return check_launch("bf prep table");
+    return div_up(std::max(div_up(maxB, (uint32_t)kBN) * kBN * 8, std::max(maxA, maxB)), 256);
 }
 
-
-
-template <class Src>
-__global__ void merge_top2_kernel(const Src batch)
+int launch_prep_table(const DevTask* tasks, uint32_t nTasks, uint32_t maxA, uint32_t maxB, hipStream_t stream)
 {
-    const DevTask& T = batch[blockIdx.z];
-    const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= T.nA || T.nSeg <= 1) return;
-    uint64_t k1 = kNoMatch, k2 = kNoMatch;
-    // segments at or past this task's train count were never written
-    const uint32_t nUsed = min(T.nSeg, (T.nB + T.segCols - 1) / T.segCols);
-    for (uint32_t s = 0; s < nUsed; s++) {
-        const uint64_t* p = T.part + ((size_t)s * T.nA + row) * 2;
-        const uint64_t o1 = p[0], o2 = p[1];
-        k2 = umin64(umax64(k1, o1), umin64(k2, o2));
-        k1 = umin64(k1, o1);
-    }
-    T.bestA[row] = k1;
-    T.secondA[row] = k2;
+    if (nTasks == 0 || (maxA == 0 && maxB == 0)) return RSFM_OK;
+    prep_train_kernel<8><<<dim3(prep_blocks(maxA, maxB), 1, nTasks), 256, 0, stream>>>(TaskTable{tasks});
+    return check_launch("bf prep table");
 }
 
 // Launch geometry shared by the size query and the launch.
@@ -685,6 +669,15 @@ struct Plan {
     uint32_t gridX = 0, nSeg = 1, segCols = kBN;
     uint32_t maxA = 0, maxB = 0;
 };
+
+// Columns per segment. Alone on its CU a workgroup takes about 6 us of its own
+// and 1 us per 64-column chunk (latency: the chip is far from full), so few row
+// blocks gain from short segments until every CU has a workgroup: one pair of
+// 1000 x 1187 took 23.0 us as four workgroups and takes 10.1 us as 36, 4096 x 4096 top-1 18.1 -> 11 us. Segments above 2048
+// columns are worth two workgroups per CU (16384 x 15411: 46.2 -> 44.8 us);
+// at 8192 x 8192 one and two per CU are equal (20.1, 20.7 us) and one merges
+// less.
+constexpr uint32_t kMinSegCols = 128;
 
 static Plan make_plan(const DevTask* t, size_t n, uint32_t maxSegCols)
 {
@@ -695,10 +688,10 @@ static Plan make_plan(const DevTask* t, size_t n, uint32_t maxSegCols)
     }
     p.gridX = div_up(p.maxA, kBM);
     if (p.maxA == 0 || p.maxB == 0) return p;
-    // aim for >= 512 workgroups (2 per CU) but keep >= 1024 columns per segment
     const uint32_t wg = p.gridX * (uint32_t)n;
-    uint32_t nSeg = div_up(512, wg);
-    nSeg = std::min(nSeg, std::max(1u, p.maxB / 1024));
+    uint32_t nSeg = div_up(256, wg);
+    if (p.maxB / nSeg > 2048) nSeg = div_up(512, wg);
+    nSeg = std::min(nSeg, std::max(1u, p.maxB / kMinSegCols));
     nSeg = std::max(nSeg, div_up(p.maxB, maxSegCols));
     uint32_t seg = div_up(p.maxB, nSeg);
     seg = div_up(seg, kBN) * kBN;
@@ -732,6 +725,21 @@ static DevTask to_dev(const rsfm_bf_task& t)
     return d;
 }
 
+// The kernels' task argument at the batch's size: a launch copies it whole, and
+// the 32-task form is 2.6 KB. With it and with the segments merged in the tile
+// instead of by a launch of its own, one pair of 1000 x 1187 matched and
+// filtered takes 29.4 us per call against 31.3 (host-bound; 17 us of kernels
+// against 31).
+template <class F>
+static int with_batch(const TaskBatch& batch, size_t n, F launch)
+{
+    constexpr int kSmall = 2;
+    if (n > (size_t)kSmall) return launch(batch);
+    ByValue<DevTask, kSmall> s{};
+    for (size_t i = 0; i < n; i++) s.t[i] = batch.t[i];
+    return launch(s);
+}
+
 // Top-1 entry points: the tile needs the train sets' staging form, which the
 // reference interface has no workspace for, so the call takes it from the
 // stream-ordered allocator (hipMallocAsync / hipFreeAsync on the same stream:
@@ -752,8 +760,7 @@ static int launch_top1(const rsfm_bf_task* tasks, size_t nbTasks, hipStream_t st
             batch.t[i].segCols = p.segCols;
             bytes += prep_bytes(batch.t[i].nA, batch.t[i].nB);
         }
-        const uint32_t prepThreads = std::max(div_up(p.maxB, (uint32_t)kBN) * kBN * 8, std::max(p.maxA, p.maxB));
-        if (prepThreads == 0) continue;
+        if (p.maxA == 0 && p.maxB == 0) continue;
         void* ws = nullptr;
         if (bytes > 0) RSFM_CHECK(check_hip(hipMallocAsync(&ws, bytes, stream), "bf match: staging workspace"));
         uint8_t* w = static_cast<uint8_t*>(ws);
@@ -761,12 +768,14 @@ static int launch_top1(const rsfm_bf_task* tasks, size_t nbTasks, hipStream_t st
             place_prep(batch.t[i], w);
             w += prep_bytes(batch.t[i].nA, batch.t[i].nB);
         }
-        prep_train_kernel<kBits><<<dim3(div_up(prepThreads, 256), 1, (uint32_t)n), 256, 0, stream>>>(batch, kInitTop1);
-        int rc = check_launch("bf prep");
-        if (rc == RSFM_OK && p.gridX > 0 && p.maxB > 0) {
-            match_top1_kernel<kBits><<<dim3(p.gridX, p.nSeg, (uint32_t)n), 512, 0, stream>>>(batch);
-            rc = check_launch("bf match");
-        }
+        int rc = with_batch(batch, n, [&](const auto& src) {
+            typedef std::decay_t<decltype(src)> Src;
+            prep_train_kernel<kBits, Src><<<dim3(prep_blocks(p.maxA, p.maxB), 1, (uint32_t)n), 256, 0, stream>>>(src);
+            RSFM_CHECK(check_launch("bf prep"));
+            if (p.gridX == 0 || p.maxB == 0) return RSFM_OK;
+            match_top1_kernel<kBits, Src><<<dim3(p.gridX, p.nSeg, (uint32_t)n), 512, 0, stream>>>(src);
+            return check_launch("bf match");
+        });
         if (ws != nullptr) {
             const int rf = check_hip(hipFreeAsync(ws, stream), "bf match: staging workspace release");
             if (rc == RSFM_OK) rc = rf;
@@ -779,16 +788,7 @@ static int launch_top1(const rsfm_bf_task* tasks, size_t nbTasks, hipStream_t st
 static size_t top2_workspace(const rsfm_bf_top2_task* tasks, size_t nbTasks)
 {
     size_t bytes = 0;
-    for (size_t b = 0; b < nbTasks; b += kMaxTasks) {
-        const size_t n = std::min<size_t>(kMaxTasks, nbTasks - b);
-        DevTask t[kMaxTasks];
-        for (size_t i = 0; i < n; i++) t[i] = to_dev(tasks[b + i].base);
-        const Plan p = make_plan(t, n, kMaxSegColsTop2);
-        for (size_t i = 0; i < n; i++) {
-            if (p.nSeg > 1) bytes += align_up((size_t)p.nSeg * t[i].nA * 16, 256);
-            bytes += prep_bytes(t[i].nA, t[i].nB);
-        }
-    }
+    for (size_t i = 0; i < nbTasks; i++) bytes += prep_bytes(tasks[i].base.nbDescA, tasks[i].base.nbDescB);
     return bytes;
 }
 
@@ -806,13 +806,6 @@ int launch_match_tile_grid_top2(const DevTask* tasks, const TileDesc* tiles, con
     if (maxList == 0) return RSFM_OK;
     match_tile_grid_kernel<<<maxList * kNumXcd, 512, 0, stream>>>(tasks, tiles, xcdOff);
     return check_launch("bf match tile grid");
-}
-
-int launch_merge_top2_table(const DevTask* tasks, uint32_t nTasks, uint32_t maxA, hipStream_t stream)
-{
-    if (nTasks == 0 || maxA == 0) return RSFM_OK;
-    merge_top2_kernel<<<dim3(div_up(maxA, 256), 1, nTasks), 256, 0, stream>>>(TaskTable{tasks});
-    return check_launch("bf merge table");
 }
 
 }  // namespace bf
@@ -869,39 +862,32 @@ extern "C" int rsfm_bf_match_top2(const rsfm_bf_top2_task* tasks, size_t nbTasks
             batch.t[i].segCols = p.segCols;
         }
         for (size_t i = 0; i < n; i++) {
-            if (p.nSeg > 1) {
-                batch.t[i].part = reinterpret_cast<uint64_t*>(ws);
-                ws += align_up((size_t)p.nSeg * batch.t[i].nA * 16, 256);
-            }
             place_prep(batch.t[i], ws);
             ws += prep_bytes(batch.t[i].nA, batch.t[i].nB);
         }
-        // one launch: results to "no match" where no tile writes them, and
-        // the staging form of every task's train descriptors
-        const uint32_t prepThreads = std::max(div_up(p.maxB, (uint32_t)kBN) * kBN * 8, std::max(p.maxA, p.maxB));
-        if (prepThreads == 0) continue;
-        prep_train_kernel<8><<<dim3(div_up(prepThreads, 256), 1, (uint32_t)n), 256, 0, stream>>>(batch, kInitTop2);
-        RSFM_CHECK(check_launch("bf top2 prep"));
-        if (p.gridX == 0 || p.maxB == 0) continue;
-        match_top2_kernel<<<dim3(p.gridX, p.nSeg, (uint32_t)n), 512, 0, stream>>>(batch);
-        RSFM_CHECK(check_launch("bf top2 match"));
-        if (p.nSeg > 1) {
-            merge_top2_kernel<<<dim3(div_up(p.maxA, 256), 1, (uint32_t)n), 256, 0, stream>>>(batch);
-            RSFM_CHECK(check_launch("bf top2 merge"));
-        }
+        if (p.maxA == 0 && p.maxB == 0) continue;
+        // one launch: results to "no match" where they are merged or no tile writes
+        // them, and the staging form of every task's train descriptors
+        RSFM_CHECK(with_batch(batch, n, [&](const auto& src) {
+            typedef std::decay_t<decltype(src)> Src;
+            prep_train_kernel<8, Src><<<dim3(prep_blocks(p.maxA, p.maxB), 1, (uint32_t)n), 256, 0, stream>>>(src);
+            RSFM_CHECK(check_launch("bf top2 prep"));
+            if (p.gridX == 0 || p.maxB == 0) return RSFM_OK;
+            match_top2_kernel<Src><<<dim3(p.gridX, p.nSeg, (uint32_t)n), 512, 0, stream>>>(src);
+            return check_launch("bf top2 match");
+        }));
     }
     return RSFM_OK;
 }
 
 // ---------------------------------------------------------------------------
 // rsfm_bf_match_top2_noalloc: the top-2 matcher with its workspace (train
-// staging form and segment partials) in a fixed device array instead of a
+// staging form) in a fixed device array instead of a
 // caller buffer, for callers that cannot allocate. The array is this file's
 // `scratch`; its device address is looked up once per device, with that device
 // current, and only that address is handed to kernels. Every call on one GPU
 // shares the array (calls that overlap on one GPU race); nothing in it needs
-// clearing (the preparation kernel writes the whole staging form and every
-// partial that the merge reads is written by a tile first).
+// clearing (the preparation kernel writes the whole staging form).
 namespace {
 constexpr size_t kNoAllocScratchBytes = size_t(64) << 20;
 constexpr int kMaxDevices = 64;

@@ -31,7 +31,6 @@ struct DevTask {
     uint64_t* bestA;
     uint64_t* secondA;  // top-2 only
     uint64_t* bestB;    // may be null
-    uint64_t* part;     // top-2 with several segments: [nSeg][nA][2]
     uint32_t nSeg;      // column segments of this task (1: results written directly)
     uint32_t segCols;   // columns per segment (multiple of kBN, <= kMaxSegColsTop2)
     // staging form of B, written by the preparation kernel: w = b - 128
@@ -63,11 +62,9 @@ int launch_match_tile_grid_top2(const DevTask* tasks, const TileDesc* tiles, con
 size_t prep_bytes(uint32_t nA, uint32_t nB);
 // point W, NB and colMin of t into ws (prep_bytes(t.nA, t.nB) bytes)
 void place_prep(DevTask& t, uint8_t* ws);
-// staging form of B for the listed tasks (W, NB set, colMin cleared); maxB = largest nB
-int launch_prep_table(const DevTask* tasks, uint32_t nTasks, uint32_t maxB, hipStream_t stream);
-
-// merge of the segment partials of the listed tasks (all with nSeg > 1)
-int launch_merge_top2_table(const DevTask* tasks, uint32_t nTasks, uint32_t maxA, hipStream_t stream);
+// staging form of B for the listed tasks (W, NB set, colMin cleared), results
+// that are merged or that no tile writes to "no match"; maxA, maxB = largest nA, nB
+int launch_prep_table(const DevTask* tasks, uint32_t nTasks, uint32_t maxA, uint32_t maxB, hipStream_t stream);
 }  // namespace bf
 
 namespace aux {

@@ -18,11 +18,10 @@
 //    pairs run largest first. Tile width (segment columns) and the persistent
 //    grid are chosen by an autotuner that times the candidates on the batch
 //    itself (HIP events, best of three) unless the caller fixes them.
-//  * The stages (fill, match, segment merge, ratio/cross-check filter with
-//    keypoint gather, seeded sampler, 8-point fit + scoring, best model and
-//    inlier mask) are captured once into a HIP graph on a private stream;
-//    rsfm_pipeline_run launches that graph. Buffers are cleared by a fill
-//    kernel (no memset nodes).
+//  * The stages (preparation, which also clears the results, match,
+//    ratio/cross-check filter with keypoint gather, seeded sampler, 8-point fit +
+//    scoring, best model and inlier mask) are captured once into a HIP graph on
+//    a private stream; rsfm_pipeline_run launches that graph (no memset nodes).
 //  * Pairs that carry lens distortion have their gathered keypoint pairs
 //    undistorted in place right after the filter (one launch over a device
 //    table), as the reference's makePtPair does before solving.
@@ -44,23 +43,6 @@
 #include <numeric>
 #include <vector>
 
-namespace rsfm_amd {
-namespace pipe {
-
-struct FillRange {
-    uint64_t* p;
-    uint32_t n;
-};
-
-__global__ void fill_kernel(const FillRange* __restrict__ ranges, uint64_t value)
-{
-    const FillRange r = ranges[blockIdx.y];
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < r.n; i += gridDim.x * blockDim.x) r.p[i] = value;
-}
-
-}  // namespace pipe
-}  // namespace rsfm_amd
-
 using namespace rsfm_amd;
 
 struct rsfm_pipeline {
@@ -70,8 +52,6 @@ struct rsfm_pipeline {
     uint8_t* arena = nullptr;
     // device tables
     bf::DevTask* dTasks = nullptr;
-    bf::DevTask* dMerge = nullptr;
-    uint32_t nMerge = 0, maxAMerge = 0;
     bf::TileDesc* dTiles = nullptr;
     uint32_t* dXcdOff = nullptr;
     size_t tileCap = 0;
@@ -84,12 +64,8 @@ struct rsfm_pipeline {
     rmf::BatchTask* dRmf = nullptr;  // affine match filter stage
     rmf::BatchParams rmfParams{};
     uint32_t rmfCols = 0, rmfRows = 0;
-    pipe::FillRange* dFill = nullptr;
-    uint32_t nFill = 0, maxFill = 0;
-    uint64_t* dPart = nullptr;
-    size_t partCap = 0;
     uint8_t* dPrep = nullptr;  // staging form of every pair's train descriptors
-    uint32_t maxPrepB = 0;
+    uint32_t maxA = 0, maxB = 0;
     // chosen tiling
     uint32_t segCols = 0, wgPerXcd = 0, nTiles = 0, maxList = 0;
     float tunedMs = 0.f;
@@ -112,24 +88,16 @@ struct rsfm_pipeline {
 
 namespace {
 
-uint32_t tasks_max_a(const std::vector<rsfm_pipeline_pair>& p)
-{
-    uint32_t m = 0;
-    for (auto& x : p) m = std::max(m, x.nA);
-    return m;
-}
-
-// Host plan for one segment width: per-pair task descriptors (segments, part
-// offsets), the tile table in XCD lists and the total partial-buffer size.
+// Host plan for one segment width: per-pair task descriptors, the tile table in
+// XCD lists.
 struct Plan {
     std::vector<bf::DevTask> tasks;
     std::vector<bf::TileDesc> tiles;
     std::vector<uint32_t> xcdOff;
-    size_t partWords = 0;
     size_t prepBytes = 0;
 };
 
-Plan make_plan(const std::vector<rsfm_pipeline_pair>& pairs, uint32_t segCols, uint64_t* part, uint8_t* prep)
+Plan make_plan(const std::vector<rsfm_pipeline_pair>& pairs, uint32_t segCols, uint8_t* prep)
 {
     Plan pl;
     const size_t P = pairs.size();
@@ -147,10 +115,6 @@ Plan make_plan(const std::vector<rsfm_pipeline_pair>& pairs, uint32_t segCols, u
         t.bestB = reinterpret_cast<uint64_t*>(x.bestB);
         t.segCols = segCols;
         t.nSeg = std::max(1u, div_up(x.nB, segCols));
-        if (t.nSeg > 1) {
-            t.part = part ? part + pl.partWords : nullptr;
-            pl.partWords += (size_t)t.nSeg * x.nA * 2;
-        }
         if (prep) bf::place_prep(t, prep + pl.prepBytes);
         pl.prepBytes += bf::prep_bytes(x.nA, x.nB);
     }
@@ -188,44 +152,27 @@ int upload(void* dst, const void* src, size_t bytes)
     return check_hip(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice), "pipeline upload");
 }
 
-// fill + match + merge of the current plan on stream s
+// preparation + match of the current plan on stream s
 int enqueue_match(rsfm_pipeline* pl, hipStream_t s)
 {
-    if (pl->nFill) {
-        pipe::fill_kernel<<<dim3(std::min<uint32_t>(div_up(pl->maxFill, 256), 64), pl->nFill), 256, 0, s>>>(pl->dFill,
-                                                                                                         kNoMatch);
-        RSFM_CHECK(check_launch("pipeline fill"));
-    }
+    RSFM_CHECK(bf::launch_prep_table(pl->dTasks, (uint32_t)pl->pairs.size(), pl->maxA, pl->maxB, s));
     if (pl->nTiles) {
-        RSFM_CHECK(bf::launch_prep_table(pl->dTasks, (uint32_t)pl->pairs.size(), pl->maxPrepB, s));
         if (pl->wgPerXcd == RSFM_PIPELINE_WG_PER_TILE)
             RSFM_CHECK(bf::launch_match_tile_grid_top2(pl->dTasks, pl->dTiles, pl->dXcdOff, pl->maxList, s));
         else
             RSFM_CHECK(bf::launch_match_tiles_top2(pl->dTasks, pl->dTiles, pl->dXcdOff, pl->wgPerXcd * kNumXcd, s));
     }
-    RSFM_CHECK(bf::launch_merge_top2_table(pl->dMerge, pl->nMerge, pl->maxAMerge, s));
     return RSFM_OK;
 }
 
 // upload the plan for segment width segCols
 int apply_plan(rsfm_pipeline* pl, uint32_t segCols)
 {
-    Plan p = make_plan(pl->pairs, segCols, pl->dPart, pl->dPrep);
-    RSFM_RETURN_IF(p.partWords > pl->partCap, RSFM_ERR_INVALID, "pipeline: partial buffer too small");
+    Plan p = make_plan(pl->pairs, segCols, pl->dPrep);
     RSFM_RETURN_IF(p.tiles.size() > pl->tileCap, RSFM_ERR_INVALID, "pipeline: tile table too small");
     RSFM_CHECK(upload(pl->dTasks, p.tasks.data(), p.tasks.size() * sizeof(bf::DevTask)));
     RSFM_CHECK(upload(pl->dTiles, p.tiles.data(), p.tiles.size() * sizeof(bf::TileDesc)));
     RSFM_CHECK(upload(pl->dXcdOff, p.xcdOff.data(), p.xcdOff.size() * sizeof(uint32_t)));
-    std::vector<bf::DevTask> merge;
-    uint32_t maxA = 0;
-    for (auto& t : p.tasks)
-        if (t.nSeg > 1 && t.nA > 0) {
-            merge.push_back(t);
-            maxA = std::max(maxA, t.nA);
-        }
-    RSFM_CHECK(upload(pl->dMerge, merge.data(), merge.size() * sizeof(bf::DevTask)));
-    pl->nMerge = (uint32_t)merge.size();
-    pl->maxAMerge = maxA;
     pl->segCols = segCols;
     pl->nTiles = (uint32_t)p.tiles.size();
     pl->maxList = 0;
@@ -395,25 +342,11 @@ extern "C" int rsfm_pipeline_create(const rsfm_pipeline_pair* pairs, size_t nbPa
     if (rc == RSFM_OK) rc = check_hip(hipEventCreateWithFlags(&pl->done, hipEventDisableTiming), "pipeline event");
     if (rc != RSFM_OK) return fail_out(rc);
 
-    // sizes: the finest candidate segment width bounds tiles and partials
+    // sizes: the finest candidate segment width bounds the tiles
     const uint32_t P = (uint32_t)nbPairs;
     const uint32_t minSeg = cfg->segCols ? cfg->segCols : 1024;
-    Plan worst = make_plan(pl->pairs, minSeg, nullptr, nullptr);
+    Plan worst = make_plan(pl->pairs, minSeg, nullptr);
     pl->tileCap = std::max<size_t>(1, worst.tiles.size());
-    pl->partCap = worst.partWords;
-    std::vector<pipe::FillRange> fill;
-    uint32_t maxFill = 0;
-    for (auto& x : pl->pairs) {
-        if (x.nA) {
-            fill.push_back({reinterpret_cast<uint64_t*>(x.bestA), x.nA});
-            fill.push_back({reinterpret_cast<uint64_t*>(x.secondA), x.nA});
-        }
-        if (x.nB) fill.push_back({reinterpret_cast<uint64_t*>(x.bestB), x.nB});
-        maxFill = std::max(maxFill, std::max(x.nA, x.nB));
-    }
-    pl->nFill = (uint32_t)fill.size();
-    pl->maxFill = maxFill;
-
     size_t off = 0;
     auto take = [&](size_t bytes) {
         const size_t o = off;
@@ -421,7 +354,6 @@ extern "C" int rsfm_pipeline_create(const rsfm_pipeline_pair* pairs, size_t nbPa
         return o;
     };
     const size_t oTasks = take(P * sizeof(bf::DevTask));
-    const size_t oMerge = take(P * sizeof(bf::DevTask));
     const size_t oTiles = take(pl->tileCap * sizeof(bf::TileDesc));
     const size_t oXcd = take((kNumXcd + 1) * sizeof(uint32_t));
     const size_t oFilter = take(P * sizeof(aux::FilterTask));
@@ -453,8 +385,6 @@ extern "C" int rsfm_pipeline_create(const rsfm_pipeline_pair* pairs, size_t nbPa
     const size_t oUnd = take(P * sizeof(undist::PairTask));
     const size_t oPoseF = take(P * sizeof(pose::DevTask));
     const size_t oPoseH = take(P * sizeof(pose::DevTask));
-    const size_t oFill = take(std::max<size_t>(1, fill.size()) * sizeof(pipe::FillRange));
-    const size_t oPart = take(std::max<size_t>(1, pl->partCap) * sizeof(uint64_t));
     const size_t oPrep = take(std::max<size_t>(1, worst.prepBytes));
     // 8-point solver: every hypothesis' model, so the best-model kernel reads
     // the winner instead of refitting it on one lane
@@ -463,7 +393,6 @@ extern "C" int rsfm_pipeline_create(const rsfm_pipeline_pair* pairs, size_t nbPa
     rc = check_hip(hipMalloc(reinterpret_cast<void**>(&pl->arena), off), "pipeline workspace");
     if (rc != RSFM_OK) return fail_out(rc);
     pl->dTasks = reinterpret_cast<bf::DevTask*>(pl->arena + oTasks);
-    pl->dMerge = reinterpret_cast<bf::DevTask*>(pl->arena + oMerge);
     pl->dTiles = reinterpret_cast<bf::TileDesc*>(pl->arena + oTiles);
     pl->dXcdOff = reinterpret_cast<uint32_t*>(pl->arena + oXcd);
     pl->dFilter = reinterpret_cast<aux::FilterTask*>(pl->arena + oFilter);
@@ -480,12 +409,12 @@ extern "C" int rsfm_pipeline_create(const rsfm_pipeline_pair* pairs, size_t nbPa
     pl->dUnd = reinterpret_cast<undist::PairTask*>(pl->arena + oUnd);
     pl->dPoseF = reinterpret_cast<pose::DevTask*>(pl->arena + oPoseF);
     pl->dPoseH = reinterpret_cast<pose::DevTask*>(pl->arena + oPoseH);
-    pl->dFill = reinterpret_cast<pipe::FillRange*>(pl->arena + oFill);
-    pl->dPart = reinterpret_cast<uint64_t*>(pl->arena + oPart);
     pl->dPrep = pl->arena + oPrep;
     float* dModels = reinterpret_cast<float*>(pl->arena + oModels);
-    for (auto& x : pl->pairs)
-        if (x.nA > 0 && x.nB > 0) pl->maxPrepB = std::max(pl->maxPrepB, x.nB);
+    for (auto& x : pl->pairs) {
+        pl->maxA = std::max(pl->maxA, x.nA);
+        pl->maxB = std::max(pl->maxB, x.nB);
+    }
 
     std::vector<aux::FilterTask> ft(P);
     std::vector<ransac::SampleTask> st(P);
@@ -564,8 +493,7 @@ extern "C" int rsfm_pipeline_create(const rsfm_pipeline_pair* pairs, size_t nbPa
         (rc = upload(pl->dDg, dg.data(), dg.size() * sizeof(degensac::DevTask))) != RSFM_OK ||
         (rc = upload(pl->dUnd, ud.data(), ud.size() * sizeof(undist::PairTask))) != RSFM_OK ||
         (rc = upload(pl->dPoseF, pf.data(), pf.size() * sizeof(pose::DevTask))) != RSFM_OK ||
-        (rc = upload(pl->dPoseH, ph.data(), ph.size() * sizeof(pose::DevTask))) != RSFM_OK ||
-        (rc = upload(pl->dFill, fill.data(), fill.size() * sizeof(pipe::FillRange))) != RSFM_OK)
+        (rc = upload(pl->dPoseH, ph.data(), ph.size() * sizeof(pose::DevTask))) != RSFM_OK)
         return fail_out(rc);
     pl->nUnd = (uint32_t)ud.size();
     pl->nPoseF = (uint32_t)pf.size();
