@@ -160,6 +160,13 @@ int rsfm_cashash_compute_bucket_bound(uint32_t* lower, uint32_t* upper, uint32_t
 int rsfm_cashash_build_buckets(const uint8_t* bucketIndices, uint32_t nbDesc, uint32_t* idxAllocator, uint32_t* buckets,
                                hipStream_t stream);
 
+/* hash, bucket bounds and buckets of one image in two launches: the same codes,
+ * remap (192 channels), ends, buckets (as sets) and largest bucket as the
+ * separate entry points above give. At most 65536 descriptors. */
+int rsfm_cashash_register(const int8_t* weights, const int32_t* bias, uint32_t nbChannels, const void* desc,
+                          uint32_t nbDesc, uint8_t* bucketIndices, uint32_t* remap, uint32_t* bucketEnds,
+                          uint32_t* buckets, uint32_t* maxBucketSize, hipStream_t stream);
+
 /* cashash::ImageDesc (cascadeHash.h:60-92), 32 B */
 typedef struct rsfm_cashash_image {
     const void* desc;

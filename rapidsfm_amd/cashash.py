@@ -22,6 +22,11 @@ class CasHashRerankImage(ctypes.Structure):
                 ("buckets", c_void_p), ("nbDesc", c_u32)]
 
 
+# most descriptors of an image that rsfm_cashash_register takes
+INDEX_MAX = 65536
+
+bind_extra("rsfm_cashash_register", c_int,
+           [c_void_p, c_void_p, c_u32, c_void_p, c_u32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p])
 bind_extra("rsfm_cashash_find_best_match_rerank", c_int, [c_void_p, c_void_p, c_void_p, c_u32, c_u32, c_u32, c_void_p])
 bind_extra("rsfm_cashash_accumulate_desc", c_int, [c_void_p, c_void_p, c_int, c_void_p, c_u32, c_void_p])
 bind_extra("rsfm_cashash_compute_bias", c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_u64, c_u32, c_void_p])
@@ -94,6 +99,17 @@ def build_buckets(codes, lower, stream=None):
 def register_image(desc, weights, bias, stream=None):
     """hash, histogram, bounds and buckets of one image (the cascade-hash part of
     BruteForceMatcher::registerImage). Returns a dict usable by find_best_match."""
+    n, dev, nch = desc.shape[0], desc.device, weights.shape[0]
+    if n <= INDEX_MAX and nch in (64, 192):
+        codes = torch.empty((n, 8), dtype=torch.uint8, device=dev)
+        remap = torch.empty((n, 4), dtype=torch.int32, device=dev) if nch == 192 else None
+        up = torch.empty((8, 256), dtype=torch.int32, device=dev)
+        buckets = torch.empty((8, n), dtype=torch.int32, device=dev)
+        mx = torch.empty(1, dtype=torch.int32, device=dev)
+        check(lib.rsfm_cashash_register(_ptr(weights), _ptr(bias), nch, _ptr(desc), n, _ptr(codes),
+                                        _ptr(remap) if remap is not None else None, _ptr(up), _ptr(buckets), _ptr(mx),
+                                        _stream(stream)), "register")
+        return {"desc": desc, "codes": codes, "remap": remap, "ends": up, "buckets": buckets, "n": n, "max_bucket": mx}
     codes, remap, _ = compute_hash(weights, bias, desc, stream=stream)
     hist = build_histogram(codes, stream)
     lo, up, mx = bucket_bounds(hist, stream)

@@ -109,21 +109,22 @@ __global__ void bias_kernel(int32_t* __restrict__ bias, const int8_t* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// hash: one wave per 32 descriptors, all channel blocks of 32
-constexpr int kHashWaves = 4;
+// hash: a workgroup takes 32 descriptors, each of its waves two channel blocks
+// of 32 (the code blocks, then pairs of remap words), so 8K descriptors run on
+// all CUs and a wave waits for 8 KB of weights instead of 24: 6.7 -> 4.3 us.
+// `clear` (optional) is set to zero.
+constexpr int kHashBlocksPerWave = 2;
 
 template <int kChBlocks>
-__global__ __launch_bounds__(kHashWaves * 64) void hash_kernel(const int8_t* __restrict__ w, const int32_t* __restrict__ bias,
-                                                                const uint8_t* __restrict__ desc, uint32_t n,
-                                                                uint32_t* __restrict__ codes, uint32_t* __restrict__ remap,
-                                                                uint32_t* __restrict__ hist)
+__global__ __launch_bounds__(kChBlocks / kHashBlocksPerWave * 64) void hash_kernel(
+    const int8_t* __restrict__ w, const int32_t* __restrict__ bias, const uint8_t* __restrict__ desc, uint32_t n,
+    uint32_t* __restrict__ codes, uint32_t* __restrict__ remap, uint32_t* __restrict__ hist, uint32_t* __restrict__ clear)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, hi = lane >> 5;
-    const uint32_t rowBase = (blockIdx.x * kHashWaves + wave) * 32;
-    if (rowBase >= n) return;
-    const uint32_t row = rowBase + l32;
+    const uint32_t row = blockIdx.x * 32 + l32;
     const bool valid = row < n;
+    if (clear != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
     v4i aop[4];
 #pragma unroll
     for (int kc = 0; kc < 4; kc++) {
@@ -133,10 +134,10 @@ __global__ __launch_bounds__(kHashWaves * 64) void hash_kernel(const int8_t* __r
         for (int q = 0; q < 4; q++) x[q] = (int)(((uint32_t)x[q] >> 1) & 0x7F7F7F7Fu);
         aop[kc] = x;
     }
-    uint32_t myWord[kChBlocks];
+    uint32_t myWord[kHashBlocksPerWave];
 #pragma unroll
-    for (int cb = 0; cb < kChBlocks; cb++) {
-        const int ch = cb * 32 + l32;
+    for (int cb = 0; cb < kHashBlocksPerWave; cb++) {
+        const int ch = (wave * kHashBlocksPerWave + cb) * 32 + l32;
         v16i acc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int kc = 0; kc < 4; kc++) {
@@ -156,19 +157,15 @@ __global__ __launch_bounds__(kHashWaves * 64) void hash_kernel(const int8_t* __r
         }
         myWord[cb] = mine;
     }
-    if (valid && hi == 0) {
-        codes[(size_t)row * 2 + 0] = myWord[0];
-        codes[(size_t)row * 2 + 1] = myWord[1];
-        if constexpr (kChBlocks > 2) {
-            if (remap) {
+    if (!valid || hi != 0) return;
+    if (wave > 0) {
+        if (remap) *reinterpret_cast<uint2*>(remap + (size_t)row * 4 + (wave - 1) * 2) = make_uint2(myWord[0], myWord[1]);
+        return;
+    }
+    *reinterpret_cast<uint2*>(codes + (size_t)row * 2) = make_uint2(myWord[0], myWord[1]);
+    if (hist) {
 #pragma unroll
-                for (int r = 0; r < 4; r++) remap[(size_t)row * 4 + r] = myWord[2 + r];
-            }
-        }
-        if (hist) {
-#pragma unroll
-            for (int s = 0; s < 8; s++) atomicAdd(&hist[s * 256 + ((myWord[s >> 2] >> (8 * (s & 3))) & 0xFF)], 1u);
-        }
+        for (int s = 0; s < 8; s++) atomicAdd(&hist[s * 256 + ((myWord[s >> 2] >> (8 * (s & 3))) & 0xFF)], 1u);
     }
 }
 
@@ -273,6 +270,81 @@ __global__ __launch_bounds__(kBuildThreads) void buckets_kernel(const uint8_t* _
             buckets[(size_t)s * n + slot] = d;
         }
     }
+}
+
+// Histogram, bounds and buckets of one image in one launch: a workgroup per
+// scheme, whose 16 waves take contiguous parts of the descriptors. Each wave
+// counts in a histogram of its own (a skewed bucket is contended by one wave
+// only), a scan over buckets and waves turns the counts into slot cursors, and
+// a second pass over the codes fills the buckets: no global atomics, nothing to
+// clear. 8K descriptors: 9 us instead of 17.5 us of five launches (two of
+// them clears and copies). One workgroup per scheme is the slower form beyond
+// kIndexMax descriptors.
+constexpr int kIndexWaves = 16;
+constexpr uint32_t kIndexMax = 65536;
+
+__global__ __launch_bounds__(kIndexWaves * 64) void index_kernel(const uint8_t* __restrict__ codes, uint32_t n,
+                                                                 uint32_t* __restrict__ ends, uint32_t* __restrict__ buckets,
+                                                                 uint32_t* __restrict__ maxBucket)
+{
+    __shared__ uint32_t sCnt[kIndexWaves][kBuckets];
+    __shared__ uint32_t sScan[4], sMax[4];
+    const uint32_t s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (uint32_t i = tid; i < kIndexWaves * kBuckets; i += kIndexWaves * 64) (&sCnt[0][0])[i] = 0;
+    const uint32_t part = ((n + kIndexWaves - 1) / kIndexWaves + 63u) & ~63u;
+    const uint32_t beg = min(n, wave * part), end = min(n, beg + part);
+    constexpr int kBatch = 8;
+    // the wave's codes, kBatch x 64 at a time with their loads issued together
+    auto walk = [&](auto use) {
+        for (uint32_t d0 = beg; d0 < end; d0 += 64 * kBatch) {
+            uint32_t c[kBatch];
+#pragma unroll
+            for (int k = 0; k < kBatch; k++) {
+                const uint32_t d = d0 + k * 64 + lane;
+                c[k] = d < end ? codes[(size_t)d * 8 + s] : 0u;
+            }
+#pragma unroll
+            for (int k = 0; k < kBatch; k++) {
+                const uint32_t d = d0 + k * 64 + lane;
+                if (d < end) use(d, c[k]);
+            }
+        }
+    };
+    __syncthreads();
+    walk([&](uint32_t, uint32_t c) { atomicAdd(&sCnt[wave][c], 1u); });
+    __syncthreads();
+    uint32_t total = 0, inc = 0;
+    if (tid < kBuckets) {
+#pragma unroll
+        for (int w = 0; w < kIndexWaves; w++) {
+            const uint32_t c = sCnt[w][tid];
+            sCnt[w][tid] = total;
+            total += c;
+        }
+        inc = total;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)inc, o);
+            if (lane >= (uint32_t)o) inc += y;
+        }
+        uint32_t mx = total;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
+        if (lane == 63) {
+            sScan[wave] = inc;
+            sMax[wave] = mx;
+        }
+    }
+    __syncthreads();
+    if (tid < kBuckets) {
+        for (uint32_t w = 0; w < wave; w++) inc += sScan[w];
+        ends[s * kBuckets + tid] = inc;
+#pragma unroll
+        for (int w = 0; w < kIndexWaves; w++) sCnt[w][tid] += inc - total;
+        if (tid == 0 && maxBucket) atomicMax(maxBucket, max(max(sMax[0], sMax[1]), max(sMax[2], sMax[3])));
+    }
+    __syncthreads();
+    walk([&](uint32_t d, uint32_t c) { buckets[(size_t)s * n + atomicAdd(&sCnt[wave][c], 1u)] = d; });
 }
 
 // ---------------------------------------------------------------------------
@@ -811,7 +883,8 @@ extern "C" int rsfm_cashash_compute_bias(int32_t* bias, const int8_t* weights, c
 }
 
 static int launch_hash(const int8_t* weights, const int32_t* bias, const void* desc, uint32_t nbDesc, uint8_t* bucketIndices,
-                       uint32_t* remap, uint32_t* histogram, hipStream_t stream, bool withRemap)
+                       uint32_t* remap, uint32_t* histogram, hipStream_t stream, bool withRemap,
+                       uint32_t* clear = nullptr)
 {
     RSFM_RETURN_IF(weights == nullptr || bias == nullptr, RSFM_ERR_INVALID, "compute_hash: weights/bias null");
     RSFM_RETURN_IF(nbDesc > 0 && (desc == nullptr || bucketIndices == nullptr), RSFM_ERR_INVALID,
@@ -825,15 +898,33 @@ static int launch_hash(const int8_t* weights, const int32_t* bias, const void* d
         RSFM_CHECK(check_launch("compute_hash histogram init"));
     }
     if (nbDesc == 0) return RSFM_OK;
-    const uint32_t blocks = div_up(nbDesc, 32 * cashash::kHashWaves);
+    const uint32_t blocks = div_up(nbDesc, 32);
     uint32_t* codes = reinterpret_cast<uint32_t*>(bucketIndices);
     if (withRemap)
-        cashash::hash_kernel<6><<<blocks, cashash::kHashWaves * 64, 0, stream>>>(
-            weights, bias, static_cast<const uint8_t*>(desc), nbDesc, codes, remap, histogram);
+        cashash::hash_kernel<6><<<blocks, 192, 0, stream>>>(weights, bias, static_cast<const uint8_t*>(desc), nbDesc, codes,
+                                                            remap, histogram, clear);
     else
-        cashash::hash_kernel<2><<<blocks, cashash::kHashWaves * 64, 0, stream>>>(
-            weights, bias, static_cast<const uint8_t*>(desc), nbDesc, codes, nullptr, histogram);
+        cashash::hash_kernel<2><<<blocks, 64, 0, stream>>>(weights, bias, static_cast<const uint8_t*>(desc), nbDesc, codes,
+                                                           nullptr, histogram, clear);
     return check_launch("compute_hash");
+}
+
+extern "C" int rsfm_cashash_register(const int8_t* weights, const int32_t* bias, uint32_t nbChannels, const void* desc,
+                                     uint32_t nbDesc, uint8_t* bucketIndices, uint32_t* remap, uint32_t* bucketEnds,
+                                     uint32_t* buckets, uint32_t* maxBucketSize, hipStream_t stream)
+{
+    RSFM_RETURN_IF(nbChannels != 64 && nbChannels != 192, RSFM_ERR_INVALID, "register: nbChannels must be 64 or 192");
+    RSFM_RETURN_IF(nbDesc > cashash::kIndexMax, RSFM_ERR_UNSUPPORTED, "register: at most 65536 descriptors");
+    RSFM_RETURN_IF(bucketEnds == nullptr || maxBucketSize == nullptr || (nbDesc > 0 && buckets == nullptr),
+                   RSFM_ERR_INVALID, "register: null pointer");
+    if (nbDesc == 0) {
+        cashash::zero_u32_kernel<<<1, 64, 0, stream>>>(maxBucketSize, 1);
+        RSFM_CHECK(check_launch("register"));
+    }
+    RSFM_CHECK(launch_hash(weights, bias, desc, nbDesc, bucketIndices, remap, nullptr, stream, nbChannels == 192, maxBucketSize));
+    cashash::index_kernel<<<cashash::kSchemes, cashash::kIndexWaves * 64, 0, stream>>>(bucketIndices, nbDesc, bucketEnds,
+                                                                                       buckets, maxBucketSize);
+    return check_launch("register index");
 }
 
 extern "C" int rsfm_cashash_compute_hash_bucket_only(const int8_t* weights, const int32_t* bias, const void* desc,
