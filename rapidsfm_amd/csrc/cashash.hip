@@ -744,18 +744,17 @@ __global__ __launch_bounds__(256) void rerank_recs_kernel(const RecBatch batch, 
     im.recRemap[x] = im.remap[j];
 }
 
-template <int kKeep>
-__global__ __launch_bounds__(kRerankWaves * 64) void rerank_kernel(const RerankBatch batch, uint32_t nSchemes)
+// The kKeep smallest (Hamming distance << 24 | index) keys of query qi's bucket
+// union into sel, every lane keeping the kList smallest of the records it meets.
+// False when a lane's whole list was selected: it may have dropped another.
+template <int kKeep, int kList>
+__device__ __forceinline__ bool rerank_select(const RerankTask& T, uint64_t qc, const uint4& qr, uint32_t nSchemes,
+                                              uint32_t (&sel)[kKeep])
 {
-    const RerankTask& T = batch.t[blockIdx.y];
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t qi = blockIdx.x * kRerankWaves + (threadIdx.x >> 6);
-    if (qi >= T.q.n) return;
-    const uint64_t qc = T.q.codes[qi];
-    const uint4 qr = T.q.remap[qi];
-    uint32_t top[kKeep];
+    uint32_t top[kList];
 #pragma unroll
-    for (int k = 0; k < kKeep; k++) top[k] = ~0u;
+    for (int k = 0; k < kList; k++) top[k] = ~0u;
     for (uint32_t s = 0; s < nSchemes; s++) {
         const uint32_t code = (uint32_t)(qc >> (8 * s)) & 0xFF;
         const uint32_t end = T.t.ends[s * 256 + code];
@@ -780,14 +779,14 @@ __global__ __launch_bounds__(kRerankWaves * 64) void rerank_kernel(const RerankB
                 const uint32_t h = (uint32_t)(__popc(r.x ^ qr.x) + __popc(r.y ^ qr.y) + __popc(r.z ^ qr.z) +
                                               __popc(r.w ^ qr.w));
                 uint32_t key = (h << 24) | jj[u];
-                if (key >= top[kKeep - 1]) continue;
+                if (key >= top[kList - 1]) continue;
                 // an item met in an earlier table (same key) is listed once
                 bool dup = false;
 #pragma unroll
-                for (int k = 0; k < kKeep; k++) dup = dup || top[k] == key;
+                for (int k = 0; k < kList; k++) dup = dup || top[k] == key;
                 if (dup) continue;
 #pragma unroll
-                for (int k = 0; k < kKeep; k++) {
+                for (int k = 0; k < kList; k++) {
                     const uint32_t lo = min(top[k], key);
                     key = max(top[k], key);
                     top[k] = lo;
@@ -796,17 +795,38 @@ __global__ __launch_bounds__(kRerankWaves * 64) void rerank_kernel(const RerankB
         }
     }
     // the kKeep smallest keys of the wave, in order
-    uint32_t sel[kKeep];
+    int left = kList;
 #pragma unroll
     for (int k = 0; k < kKeep; k++) {
         const uint32_t m = wave_min_u32(top[0]);
         sel[k] = m;
         if (top[0] == m && m != ~0u) {
 #pragma unroll
-            for (int u = 0; u + 1 < kKeep; u++) top[u] = top[u + 1];
-            top[kKeep - 1] = ~0u;
+            for (int u = 0; u + 1 < kList; u++) top[u] = top[u + 1];
+            top[kList - 1] = ~0u;
+            left--;
         }
     }
+    return kList >= kKeep || !__any(left == 0);
+}
+
+// One wavefront per query. A query meets some 1800 records in its buckets, 28 a
+// lane, so nearly every record enters a list of kKeep and the list's upkeep is
+// most of the work; lists of half that hold the selection unless one lane has
+// as much of it (then the query is scanned again with whole lists).
+// 8K x 8K, six tables, both directions: 88 -> 66 us (lists of three
+// scan too many queries twice: 77 us).
+template <int kKeep>
+__global__ __launch_bounds__(kRerankWaves * 64) void rerank_kernel(const RerankBatch batch, uint32_t nSchemes)
+{
+    const RerankTask& T = batch.t[blockIdx.y];
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t qi = blockIdx.x * kRerankWaves + (threadIdx.x >> 6);
+    if (qi >= T.q.n) return;
+    const uint64_t qc = T.q.codes[qi];
+    const uint4 qr = T.q.remap[qi];
+    uint32_t sel[kKeep];
+    if (!rerank_select<kKeep, kKeep / 2>(T, qc, qr, nSchemes, sel)) rerank_select<kKeep, kKeep>(T, qc, qr, nSchemes, sel);
     // exact L2^2 of the kept candidates: lane = 8 x candidate slot + 16-byte part
     const uint32_t part = lane & 7, slot = lane >> 3;
     const uint4 a = *reinterpret_cast<const uint4*>(T.q.desc + (size_t)qi * 128 + part * 16);
@@ -1005,9 +1025,11 @@ extern "C" int rsfm_cashash_find_best_match(const rsfm_cashash_image* queries, c
         if (maxN == 0) continue;
         match_init_kernel<<<dim3(div_up(maxN, 256), 1, n), 256, 0, stream>>>(batch);
         RSFM_CHECK(check_launch("find_best_match init"));
-        // about 512 workgroups (2048 waves) per launch, each wave a few
-        // 64 x 64 blocks at 8K keypoints
-        const uint32_t perTask = std::max<uint32_t>(8u, div_up(512u, n));
+        // 768 workgroups (three per CU, all that its registers hold) per launch: a
+        // wave waits for its gathers and merges most of the time (vector issue
+        // 24% busy), so residents count; two searches of 8K x 8K over eight
+        // tables take 82 us with 512, 70 with 768, 81 with 1536
+        const uint32_t perTask = std::max<uint32_t>(8u, div_up(768u, n));
         match_kernel<<<dim3(perTask, 1, n), kMatchWaves * 64, 0, stream>>>(batch, nbSchemes);
         RSFM_CHECK(check_launch("find_best_match"));
     }
