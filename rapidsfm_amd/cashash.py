@@ -134,9 +134,7 @@ def find_best_match(queries, train, n_schemes=8, bidirectional=True, stream=None
         res[i] = CasHashResult(_ptr(bq), _ptr(bt) if bt is not None else None)
         outs.append((bq, bt))
     timg = CasHashImage(_ptr(train["desc"]), _ptr(train["ends"]), _ptr(train["buckets"]), None)
-    check(lib.rsfm_cashash_find_best_match(ctypes.cast(qimg, c_void_p), ctypes.cast(qsize, c_void_p),
-                                           ctypes.cast(ctypes.pointer(timg), c_void_p),
-                                           train["n"], ctypes.cast(res, c_void_p), nq, None, 0, n_schemes,
+    check(lib.rsfm_cashash_find_best_match(qimg, qsize, ctypes.byref(timg), train["n"], res, nq, None, 0, n_schemes,
                                            _stream(stream)), "find_best_match")
     return outs
 
@@ -164,7 +162,6 @@ def find_best_match_rerank(queries, train, n_schemes=6, keep=8, bidirectional=Tr
         res[i] = CasHashResult(_ptr(bq), _ptr(bt) if bt is not None else None)
         outs.append((bq[: q["n"]], bt[: train["n"]] if bt is not None else None))
     timg = _rerank_image(train)
-    check(lib.rsfm_cashash_find_best_match_rerank(ctypes.cast(qimg, c_void_p), ctypes.cast(ctypes.pointer(timg),
-                                                  c_void_p), ctypes.cast(res, c_void_p), nq, n_schemes, keep,
+    check(lib.rsfm_cashash_find_best_match_rerank(qimg, ctypes.byref(timg), res, nq, n_schemes, keep,
                                                   _stream(stream)), "find_best_match_rerank")
     return outs

@@ -11,7 +11,7 @@ import numpy as np
 import torch
 
 from ._abi import WSampleTask, check, lib
-from .ops import _ptr, _side, _stream
+from .ops import _ptr, _rows, _side, _stream
 
 N_PARAM = lib.rsfm_mlp_param_count()
 H = 64
@@ -105,19 +105,13 @@ class Adam:
 
 def sample_weighted(tasks, stream=None):
     """tasks: list of (weights float32 (n,), H, seed[, n_dev int32 (1,)]) -> list of (H, 8) int32 index sets."""
-    outs, keep = [], []
     arr = (WSampleTask * max(1, len(tasks)))()
+    likes = [t[0] for t in tasks]
+    outs = _rows(likes, [t[1] for t in tasks], 8, torch.int32)
+    cdfs = _rows(likes, [max(1, w.shape[0]) for w in likes], None, torch.int64)
     for i, t in enumerate(tasks):
-        w, h, seed = t[0], t[1], t[2]
-        n_dev = t[3] if len(t) > 3 else None
-        idx = torch.empty((h, 8), dtype=torch.int32, device=w.device)
-        cdf = torch.empty(max(1, w.shape[0]), dtype=torch.int64, device=w.device)
-        arr[i] = WSampleTask(idx.data_ptr() if h else None, h, w.shape[0],
-                             n_dev.data_ptr() if n_dev is not None else None,
-                             w.data_ptr() if w.numel() else None, cdf.data_ptr(), seed)
-        outs.append(idx)
-        keep.append(cdf)
-    _side(stream, *outs, *keep)
-    check(lib.rsfm_ransac_sample_weighted_batch(ctypes.cast(arr, ctypes.c_void_p), len(tasks), _stream(stream)),
-          "rsfm_ransac_sample_weighted_batch")
-    return outs
+        arr[i] = WSampleTask(_ptr(outs[i]), t[1], t[0].shape[0], _ptr(t[3]) if len(t) > 3 else 0, _ptr(t[0]),
+                             _ptr(cdfs[i]), t[2])
+    _side(stream, *outs, *cdfs)
+    check(lib.rsfm_ransac_sample_weighted_batch(arr, len(tasks), _stream(stream)), "rsfm_ransac_sample_weighted_batch")
+    return list(outs)

@@ -12,9 +12,10 @@ from ._abi import BfTask, BfTop2Task, Camera, DegensacTask, FinishTask, PoseHTas
 
 
 def _stream(stream):
+    """Raw stream handle; the current stream's without building a Stream object for it."""
     if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    return stream.cuda_stream
 
 
 def _side(stream, *tensors):
@@ -30,7 +31,19 @@ def _side(stream, *tensors):
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None and t.numel() > 0 else ctypes.c_void_p(0)
+    return t.data_ptr() if t is not None and t.numel() > 0 else 0
+
+
+def _rows(likes, counts, cols, dtype):
+    """One tensor per count, (count, cols) or (count,) for cols None, each on the device of
+    its entry of likes. The parts of a batch on one device are cut from one allocation, from
+    row numbers that are multiples of 256 so that each stays aligned: a dozen allocations
+    cost the host more than the launches they are for."""
+    shape = (lambda n: (n,)) if cols is None else (lambda n: (n, cols))  # noqa: E731
+    if len(counts) < 2 or any(t.device != likes[0].device for t in likes):
+        return [torch.empty(shape(n), dtype=dtype, device=t.device) for t, n in zip(likes, counts)]
+    sizes = [m for n in counts for m in (n, -n % 256)]
+    return torch.empty(shape(sum(sizes)), dtype=dtype, device=likes[0].device).split(sizes)[::2]
 
 
 def _check_desc(d, width=128):
@@ -77,7 +90,7 @@ def bf_match(pairs, impl="mfma", bidirectional=True, stream=None):
         tasks[i] = BfTask(a.shape[0], b.shape[0], _ptr(a), _ptr(b), _ptr(ba), _ptr(bb) if bb is not None else None, None, None)
         outs.append((ba, bb))
     fn = {"mfma": lib.rsfm_bf_match_u8, "idp": lib.rsfm_bf_match_idp_u8, "u4": lib.rsfm_bf_match_u4}[impl]
-    check(fn(ctypes.cast(tasks, ctypes.c_void_p), len(pairs), _stream(stream)), "bf_match(%s)" % impl)
+    check(fn(tasks, len(pairs), _stream(stream)), "bf_match(%s)" % impl)
     return outs
 
 
@@ -96,9 +109,8 @@ def bf_match_top2(pairs, stream=None, workspace=None):
         bb = torch.empty((b.shape[0], 2), dtype=torch.int32, device=a.device)
         tasks[i] = BfTop2Task(BfTask(a.shape[0], b.shape[0], _ptr(a), _ptr(b), _ptr(ba), _ptr(bb), None, None), _ptr(sa))
         outs.append((ba, sa, bb))
-    tp = ctypes.cast(tasks, ctypes.c_void_p)
     need = ctypes.c_size_t(0)
-    check(lib.rsfm_bf_match_top2_workspace_size(tp, len(pairs), ctypes.byref(need)), "top2 workspace size")
+    check(lib.rsfm_bf_match_top2_workspace_size(tasks, len(pairs), ctypes.byref(need)), "top2 workspace size")
     ws_ptr = 0
     if need.value > 0:
         # the library wants a 256-B aligned pointer with need bytes behind it
@@ -112,7 +124,7 @@ def bf_match_top2(pairs, stream=None, workspace=None):
             if stream is not None:
                 # the temporary is freed on return: keep it until the work on stream is done
                 workspace.record_stream(stream)
-    check(lib.rsfm_bf_match_top2(tp, len(pairs), ctypes.c_void_p(ws_ptr), need.value, _stream(stream)), "bf_match_top2")
+    check(lib.rsfm_bf_match_top2(tasks, len(pairs), ws_ptr, need.value, _stream(stream)), "bf_match_top2")
     return outs
 
 
@@ -152,7 +164,7 @@ def degensac_refine(problems, threshold_f, threshold_h, mode=0, nb_candidates=8,
                                 idx.shape[0], _ptr(o["F"]), _ptr(o["H"]), _ptr(o["result"]),
                                 _ptr(o["mask_f"]) if want_masks else None, _ptr(o["mask_h"]) if want_masks else None)
         outs.append(o)
-    check(lib.rsfm_degensac_refine(ctypes.cast(tasks, ctypes.c_void_p), len(problems), float(threshold_f),
+    check(lib.rsfm_degensac_refine(tasks, len(problems), float(threshold_f),
                                    float(threshold_h), int(mode), int(nb_candidates), int(nb_plane_samples),
                                    int(seed) & 0xFFFFFFFFFFFFFFFF, _stream(stream)), "rsfm_degensac_refine")
     return outs
@@ -182,7 +194,7 @@ def undistort_pt_pairs(problems, n_iters=2, stream=None):
         mk = lambda c, k: RealCamera(Camera(*[float(v) for v in c]), (ctypes.c_float * 5)(*[float(v) for v in k]))  # noqa: E731
         tasks[i] = UndistortTask(_ptr(pts), pts.shape[0], _ptr(ndev) if ndev is not None else None, mk(c0, k0),
                                  mk(c1, k1))
-    check(lib.rsfm_undistort_pt_pairs(ctypes.cast(tasks, ctypes.c_void_p), len(problems), int(n_iters),
+    check(lib.rsfm_undistort_pt_pairs(tasks, len(problems), int(n_iters),
                                       _stream(stream)), "rsfm_undistort_pt_pairs")
 
 
@@ -206,7 +218,7 @@ def pose_from_f(problems, front_ratio=0.95, stream=None):
                             pts.shape[0], _ptr(ndev) if ndev is not None else None,
                             _ptr(mask) if mask is not None else None, _ptr(o["poses"]), _ptr(o["result"]))
         outs.append(o)
-    check(lib.rsfm_pose_from_f(ctypes.cast(tasks, ctypes.c_void_p), len(problems), float(front_ratio), _stream(stream)),
+    check(lib.rsfm_pose_from_f(tasks, len(problems), float(front_ratio), _stream(stream)),
           "rsfm_pose_from_f")
     return outs
 
@@ -234,7 +246,7 @@ def pose_from_h(problems, front_ratio=0.95, stream=None):
                              _ptr(mask) if mask is not None else None, _ptr(o["poses"]), _ptr(o["normals"]),
                              _ptr(o["result"]))
         outs.append(o)
-    check(lib.rsfm_pose_from_h(ctypes.cast(tasks, ctypes.c_void_p), len(problems), float(front_ratio), _stream(stream)),
+    check(lib.rsfm_pose_from_h(tasks, len(problems), float(front_ratio), _stream(stream)),
           "rsfm_pose_from_h")
     return outs
 
@@ -243,7 +255,7 @@ def ransac_h4(problems, threshold, min_sep_sq=(0.0, 0.0), want_models=False, str
     """4-point homography hypotheses: problems of (pts, sampleIdx (H, 4)[, nDev]);
     the inlier test is checkProjectiveTransformation's with threshold t pixels."""
     tasks, outs = _ransac_tasks(problems, want_models)
-    check(lib.rsfm_ransac_h4(ctypes.cast(tasks, ctypes.c_void_p), len(problems), float(threshold),
+    check(lib.rsfm_ransac_h4(tasks, len(problems), float(threshold),
                              float(min_sep_sq[0]), float(min_sep_sq[1]), _stream(stream)), "rsfm_ransac_h4")
     return outs
 
@@ -282,7 +294,7 @@ def ransac_f8_finish(problems, threshold, mode=1, confidence=0.0, max_iter=5000,
                               _ptr(models) if models is not None else None, idx.shape[0], _ptr(o["F"]),
                               _ptr(o["result"]), _ptr(o["mask"]))
         outs.append(o)
-    check(lib.rsfm_ransac_f8_finish(ctypes.cast(tasks, ctypes.c_void_p), len(problems), float(threshold), int(mode),
+    check(lib.rsfm_ransac_f8_finish(tasks, len(problems), float(threshold), int(mode),
                                     float(confidence), int(max_iter), int(bool(refit)), _stream(stream)),
           "rsfm_ransac_f8_finish")
     return outs
@@ -290,29 +302,28 @@ def ransac_f8_finish(problems, threshold, mode=1, confidence=0.0, max_iter=5000,
 
 def _ransac_tasks(problems, want_models):
     tasks = (RansacTask * max(1, len(problems)))()
-    outs = []
-    for i, prob in enumerate(problems):
-        pts, idx = prob[0], prob[1]
-        ndev = prob[2] if len(prob) > 2 else None
-        n, H = pts.shape[0], idx.shape[0]
+    likes = [prob[0] for prob in problems]
+    for pts in likes:
         if pts.dtype != torch.float32 or pts.dim() != 2 or pts.shape[1] != 4 or not pts.is_contiguous():
             raise ValueError("pts must be contiguous float32 (n, 4)")
-        dev = pts.device
-        o = {
-            "counts": torch.empty(H, dtype=torch.int32, device=dev),
-            "best": torch.empty(2, dtype=torch.int32, device=dev),
-            "mask": torch.empty(n, dtype=torch.uint8, device=dev),
-            "models": torch.empty((H, 3, 3), dtype=torch.float32, device=dev) if want_models else None,
-        }
-        tasks[i] = RansacTask(_ptr(pts), n, _ptr(ndev) if ndev is not None else None, _ptr(idx), H, _ptr(o["counts"]),
-                              _ptr(o["models"]) if want_models else None, _ptr(o["best"]), _ptr(o["mask"]))
+    ns, hs = [t.shape[0] for t in likes], [prob[1].shape[0] for prob in problems]
+    counts, masks = _rows(likes, hs, None, torch.int32), _rows(likes, ns, None, torch.uint8)
+    bests = _rows(likes, [2] * len(likes), None, torch.int32)
+    models = [None] * len(likes)
+    if want_models:
+        models = [m.view(h, 3, 3) for m, h in zip(_rows(likes, hs, 9, torch.float32), hs)]
+    outs = []
+    for i, prob in enumerate(problems):
+        o = {"counts": counts[i], "best": bests[i], "mask": masks[i], "models": models[i]}
+        tasks[i] = RansacTask(_ptr(prob[0]), ns[i], _ptr(prob[2]) if len(prob) > 2 else 0, _ptr(prob[1]), hs[i],
+                              _ptr(o["counts"]), _ptr(o["models"]), _ptr(o["best"]), _ptr(o["mask"]))
         outs.append(o)
     return tasks, outs
 
 
 def _ransac(fn, name, problems, threshold, mode, min_sep_sq, want_models, stream):
     tasks, outs = _ransac_tasks(problems, want_models)
-    check(fn(ctypes.cast(tasks, ctypes.c_void_p), len(problems), float(threshold), int(mode), float(min_sep_sq[0]),
+    check(fn(tasks, len(problems), float(threshold), int(mode), float(min_sep_sq[0]),
              float(min_sep_sq[1]), _stream(stream)), name)
     return outs
 

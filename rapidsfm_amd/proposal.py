@@ -25,6 +25,7 @@ import torch
 from . import learned, synth
 from ._abi import BfTask, BfTop2Task, FilterTask, RansacTask, SampleTask, check, lib
 from ._abi import bind_extra
+from .ops import _ptr, _rows, _stream
 
 RATIO = (4, 5)  # ratio test 0.8 on distances (25 d1 < 16 d2 on squared distances)
 
@@ -155,18 +156,18 @@ def subsample(rng, gt, outlier_rate):
 
 def score(problems, threshold=1.0):
     """problems: list of (pts (n,4), idx (H,8)) -> per-hypothesis counts and best masks."""
-    tasks, outs = [], []
-    for pts, idx in problems:
-        n, H = pts.shape[0], idx.shape[0]
-        o = {"counts": torch.empty(H, dtype=torch.int32, device=pts.device),
-             "best": torch.empty(2, dtype=torch.int32, device=pts.device),
-             "mask": torch.empty(max(1, n), dtype=torch.uint8, device=pts.device)}
-        tasks.append(RansacTask(pts.data_ptr(), n, None, idx.data_ptr(), H, o["counts"].data_ptr(), None,
-                                o["best"].data_ptr(), o["mask"].data_ptr()))
+    likes = [pts for pts, _ in problems]
+    counts = _rows(likes, [idx.shape[0] for _, idx in problems], None, torch.int32)
+    masks = _rows(likes, [max(1, t.shape[0]) for t in likes], None, torch.uint8)
+    bests = _rows(likes, [2] * len(likes), None, torch.int32)
+    arr = (RansacTask * max(1, len(problems)))()
+    outs = []
+    for i, (pts, idx) in enumerate(problems):
+        o = {"counts": counts[i], "best": bests[i], "mask": masks[i]}
+        arr[i] = RansacTask(_ptr(pts), pts.shape[0], None, _ptr(idx), idx.shape[0], _ptr(counts[i]), None, _ptr(bests[i]),
+                            _ptr(masks[i]))
         outs.append(o)
-    arr = _arr(RansacTask, tasks)
-    check(lib.rsfm_ransac_f8(ctypes.cast(arr, ctypes.c_void_p), len(tasks), float(threshold), 1, 0.0, 0.0, _sp()),
-          "rsfm_ransac_f8")
+    check(lib.rsfm_ransac_f8(arr, len(problems), float(threshold), 1, 0.0, 0.0, _stream(None)), "rsfm_ransac_f8")
     return outs
 
 
