@@ -338,48 +338,58 @@ __device__ inline double bisect(const double a[4], double lo, double hi)
     return 0.5 * (lo + hi);
 }
 
-// real roots of a[3] t^3 + a[2] t^2 + a[1] t + a[0] (a[3] != 0), ascending
-__device__ inline int cubic_roots(const double a[4], double r[3])
+// intervals e[0] .. e[1], e[1] .. e[2], ... that hold at most one root each of
+// a[3] t^3 + a[2] t^2 + a[1] t + a[0] (a[3] != 0): one or three, the count returned
+__device__ inline int cubic_intervals(const double a[4], double e[4])
 {
     const double inv = 1.0 / fabs(a[3]);
     double B = fabs(a[2]) * inv;
     B = fabs(a[1]) * inv > B ? fabs(a[1]) * inv : B;
     B = fabs(a[0]) * inv > B ? fabs(a[0]) * inv : B;
     B = B + 1.0;
-    double e[4] = {-B, 0.0, 0.0, B};
-    int ne = 2;
+    e[0] = -B;
+    e[1] = B;
+    e[2] = 0.0;
+    e[3] = B;
     const double disc = a[2] * a[2] - 3.0 * a[3] * a[1];
-    if (disc > 0.0) {
-        const double sq = sqrt(disc);
-        double c1 = (-a[2] - sq) / (3.0 * a[3]), c2 = (-a[2] + sq) / (3.0 * a[3]);
-        if (c2 < c1) {
-            const double tmp = c1;
-            c1 = c2;
-            c2 = tmp;
-        }
-        e[1] = c1;
-        e[2] = c2;
-        e[3] = B;
-        ne = 4;
-    } else {
-        e[1] = B;
-    }
-    int n = 0;
-    for (int i = 0; i + 1 < ne; i++) {
-        const double lo = e[i], hi = e[i + 1];
-        const double plo = cubic_at(a, lo), phi = cubic_at(a, hi);
-        if ((plo < 0.0 && phi < 0.0) || (plo > 0.0 && phi > 0.0)) continue;
-        const double x = bisect(a, lo, hi);
-        if (n > 0 && x == r[n - 1]) continue;
-        r[n++] = x;
-    }
-    return n;
+    if (!(disc > 0.0)) return 1;
+    const double sq = sqrt(disc);
+    const double c1 = (-a[2] - sq) / (3.0 * a[3]), c2 = (-a[2] + sq) / (3.0 * a[3]);
+    e[1] = c2 < c1 ? c2 : c1;
+    e[2] = c2 < c1 ? c1 : c2;
+    return 3;
 }
 
-// pts[i] = (x0, y0, x1, y1); Fs[k] row-major, unit Frobenius; returns the count
-__device__ inline int fit7(const float4 pts[7], float Fs[3][9])
+// the root in [lo, hi], false if there is none
+__device__ inline bool interval_root(const double a[4], double lo, double hi, double& x)
 {
-    float c[4] = {0.f, 0.f, 0.f, 0.f};
+    const double plo = cubic_at(a, lo), phi = cubic_at(a, hi);
+    if ((plo < 0.0 && phi < 0.0) || (plo > 0.0 && phi > 0.0)) return false;
+    x = bisect(a, lo, hi);
+    return true;
+}
+
+// appends the next interval's root, a root that two intervals share once
+__device__ inline void append_root(double r[3], int& n, double x)
+{
+    if (n > 0 && x == r[n - 1]) return;
+    r[n++] = x;
+}
+
+// what the two null vectors of a sample leave for its models: F2 and F1 - F2 by
+// column-major vectors f[1], f[0], and the normalisation
+struct Basis7 {
+    float f[2][9], c[4], s0, s1;
+};
+
+// pts[i] = (x0, y0, x1, y1): the basis and det(F2 + t (F1 - F2)) as a cubic in t;
+// false if the sample has no model
+__device__ inline bool fit7_cubic(const float4 pts[7], Basis7& S, double a[4])
+{
+    float (&f)[2][9] = S.f;
+    float (&c)[4] = S.c;
+#pragma unroll
+    for (int k = 0; k < 4; k++) c[k] = 0.f;
 #pragma unroll
     for (int i = 0; i < 7; i++) {
         c[0] = c[0] + pts[i].x;
@@ -398,9 +408,11 @@ __device__ inline int fit7(const float4 pts[7], float Fs[3][9])
     }
     n0 = n0 / 7.f;
     n1 = n1 / 7.f;
-    if (!(n0 > 0.f) || !(n1 > 0.f)) return 0;
+    if (!(n0 > 0.f) || !(n1 > 0.f)) return false;
     const float sqrt2 = 1.41421354f;
     const float s0 = sqrt2 / n0, s1 = sqrt2 / n1;
+    S.s0 = s0;
+    S.s1 = s1;
     float M[9][7];
 #pragma unroll
     for (int i = 0; i < 7; i++) {
@@ -449,7 +461,6 @@ __device__ inline int fit7(const float4 pts[7], float Fs[3][9])
         }
     }
     // f1 = Q e8, f2 = Q e7
-    float f[2][9];
 #pragma unroll
     for (int q = 0; q < 2; q++) {
 #pragma unroll
@@ -486,7 +497,6 @@ __device__ inline int fit7(const float4 pts[7], float Fs[3][9])
             for (int cc = 0; cc < 3; cc++) G[r][cc] = F2[r][cc] + ts[q] * D[r][cc];
         d[q] = det3d(G);
     }
-    double a[4];
     a[0] = d[0];
     a[2] = 0.5 * (d[1] + d[2]) - d[0];
     const double sOdd = 0.5 * (d[1] - d[2]);
@@ -494,11 +504,24 @@ __device__ inline int fit7(const float4 pts[7], float Fs[3][9])
     a[1] = sOdd - a[3];
     double scale = fabs(a[0]);
     for (int q = 1; q < 4; q++) scale = fabs(a[q]) > scale ? fabs(a[q]) : scale;
-    if (!(scale > 0.0) || !(fabs(a[3]) > 1e-12 * scale)) return 0;
-    double roots[3];
-    const int nr = cubic_roots(a, roots);
-    const float a0 = -(s0 * c[0]), b0 = -(s0 * c[1]);
-    const float a1 = -(s1 * c[2]), b1 = -(s1 * c[3]);
+    if (!(scale > 0.0) || !(fabs(a[3]) > 1e-12 * scale)) return false;
+    return true;
+}
+
+// the models of nr roots: Fs[k] row-major, unit Frobenius; returns the count
+__device__ inline int fit7_models(const Basis7& S, const double roots[3], int nr, float Fs[3][9])
+{
+    const float s0 = S.s0, s1 = S.s1;
+    double F2[3][3], D[3][3];
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+        for (int cc = 0; cc < 3; cc++) {
+            F2[r][cc] = (double)S.f[1][3 * cc + r];
+            D[r][cc] = (double)S.f[0][3 * cc + r] - F2[r][cc];
+        }
+    const float a0 = -(s0 * S.c[0]), b0 = -(s0 * S.c[1]);
+    const float a1 = -(s1 * S.c[2]), b1 = -(s1 * S.c[3]);
     int out = 0;
     for (int k = 0; k < nr; k++) {
         float Fh[3][3];
@@ -535,6 +558,21 @@ __device__ inline int fit7(const float4 pts[7], float Fs[3][9])
         out++;
     }
     return out;
+}
+
+// pts[i] = (x0, y0, x1, y1); Fs[k] row-major, unit Frobenius; returns the count
+__device__ inline int fit7(const float4 pts[7], float Fs[3][9])
+{
+    Basis7 S;
+    double a[4], e[4], roots[3];
+    if (!fit7_cubic(pts, S, a)) return 0;
+    const int ni = cubic_intervals(a, e);
+    int nr = 0;
+    for (int i = 0; i < ni; i++) {
+        double x;
+        if (interval_root(a, e[i], e[i + 1], x)) append_root(roots, nr, x);
+    }
+    return fit7_models(S, roots, nr, Fs);
 }
 
 // Inlier tests. kMode 0 = checkEpipolarTransformation (legacy/geometry.cpp:

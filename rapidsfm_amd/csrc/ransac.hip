@@ -374,10 +374,10 @@ __device__ inline bool sane7(const float4 p[7], float s0, float s1)
     return ok;
 }
 
-__device__ inline int fit_hypothesis7(const DevTask& T, uint32_t n, uint32_t h, float s0, float s1, float Fs[kMaxF7][9])
+// the seven points of sample h, false if it is to be rejected
+__device__ inline bool load_sample7(const DevTask& T, uint32_t n, uint32_t h, float s0, float s1, float4 p[7])
 {
-    if (h >= T.H || n < 7) return 0;
-    float4 p[7];
+    if (h >= T.H || n < 7) return false;
     bool inRange = true;
 #pragma unroll
     for (int i = 0; i < 7; i++) {
@@ -385,25 +385,27 @@ __device__ inline int fit_hypothesis7(const DevTask& T, uint32_t n, uint32_t h, 
         inRange = inRange && k < n;
         p[i] = T.pts[k < n ? k : 0];
     }
-    if (!inRange || !sane7(p, s0, s1)) return 0;
-    return fgeom::fit7(p, Fs);
+    return inRange && sane7(p, s0, s1);
 }
 
 // 7-point scoring. A workgroup takes kS7Samples samples, one per lane of its
-// first two wavefronts: every such lane solves its sample (up to three F)
-// while the others scan the pair's box, and the workgroup's M models are
-// listed in LDS in sample order (a scan of the model counts). Wavefront w then
-// counts the inliers of models 16 R w .. (R = ceil(M / 128), at most three
-// blocks of 16) over all points with the matrix-core screen. A sample with one
-// real root thus takes one model slot instead of three (about 2.5 models per
-// sample with 8K-keypoint pairs). Each sample then reports its best model
-// (most inliers, the first on ties) and that count. 32 pairs x 4096 samples x
-// 1400 points on average, two-sided test: 468 -> 288 us against the exact test
-// on every point, of which the solver takes 100.
+// first two wavefronts: every such lane reduces its sample to a cubic while the
+// others scan the pair's box; the cubic's one or three root intervals are
+// bisected in FP64 by the other six wavefronts, an interval a lane (chains of up
+// to 80 dependent steps; one after the other on the sample's own lane they took
+// 30 us more); the sample's lane makes the models of the roots, up to three, and
+// the workgroup's M models are listed in LDS in sample order (a scan of the model
+// counts). Wavefront w then counts the inliers of models 16 R w .. (R = ceil(M /
+// 128), at most three blocks of 16) over all points with the matrix-core screen. A
+// sample with one real root thus takes one model slot instead of three (about 2.5
+// models per sample with 8K-keypoint pairs). Each sample then reports its best
+// model (most inliers, the first on ties) and that count. 32 pairs x 4096 samples
+// x 1400 points on average, two-sided test: 468 -> 288 us with the screen instead
+// of the exact test on every point, -> 259 with the bisections spread.
 constexpr uint32_t kS7Samples = 128;
 constexpr int kS7Waves = 8, kS7Block = 64 * kS7Waves;
 constexpr uint32_t kS7MaxModels = kS7Samples * kMaxF7;
-static_assert(kS7Samples < kS7Block && kS7Samples % 64 == 0, "samples are fitted one per lane");
+static_assert(kS7Samples % 64 == 0 && kS7Block == (1 + kMaxF7) * kS7Samples, "a lane per sample and per interval");
 
 // the wave's 16 R models (base, count of them) over all points
 template <int kMode, int R, class Sm, class Model>
@@ -426,13 +428,57 @@ __global__ __launch_bounds__(kS7Block, 4) void score7_kernel(const Src batch, fl
     const uint32_t h = wg.x * kS7Samples + tid;
     const uint32_t n = task_n(T);
     __shared__ screen::Smem<kS7Waves, 1> S;  // two workgroups per CU
-    __shared__ float sF[9][kS7MaxModels];
+    // the cubics and their roots, then the models
+    union Fit {
+        struct {
+            double a[4][kS7Samples], e[4][kS7Samples], root[kMaxF7][kS7Samples];
+            uint8_t intervals[kS7Samples], has[kMaxF7][kS7Samples];
+        } s;
+        float F[9][kS7MaxModels];
+    };
+    __shared__ Fit fit;
+    float (&sF)[9][kS7MaxModels] = fit.F;
     __shared__ uint32_t sCnt[kS7MaxModels];
     __shared__ uint32_t sWaveModels[kS7Samples / 64];
     for (uint32_t k = tid; k < kS7MaxModels; k += kS7Block) sCnt[k] = 0u;
-    float Fw[kMaxF7][9];  // written by the solver with a running index
-    const int nm = tid < kS7Samples ? fit_hypothesis7(T, n, h, s0, s1, Fw) : 0;
-    if (tid >= kS7Samples) box_scan(S, T.pts, n, tid - kS7Samples, kS7Block - kS7Samples);
+    fgeom::Basis7 basis;
+    int ni = 0;
+    if (tid < kS7Samples) {
+        float4 p[7];
+        double a[4], e[4];
+        if (load_sample7(T, n, h, s0, s1, p) && fgeom::fit7_cubic(p, basis, a)) {
+            ni = fgeom::cubic_intervals(a, e);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                fit.s.a[k][tid] = a[k];
+                fit.s.e[k][tid] = e[k];
+            }
+        }
+        fit.s.intervals[tid] = (uint8_t)ni;
+    } else {
+        box_scan(S, T.pts, n, tid - kS7Samples, kS7Block - kS7Samples);
+    }
+    __syncthreads();
+    if (tid >= kS7Samples) {
+        const uint32_t i = tid / kS7Samples - 1, s = tid % kS7Samples;
+        if (i < fit.s.intervals[s]) {
+            double a[4], x = 0.0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) a[k] = fit.s.a[k][s];
+            fit.s.has[i][s] = fgeom::interval_root(a, fit.s.e[i][s], fit.s.e[i + 1][s], x);
+            fit.s.root[i][s] = x;
+        }
+    }
+    __syncthreads();
+    float Fw[kMaxF7][9];  // written with a running index
+    int nm = 0;
+    if (ni > 0) {
+        double roots[kMaxF7];
+        int nr = 0;
+        for (int i = 0; i < ni; i++)
+            if (fit.s.has[i][tid]) fgeom::append_root(roots, nr, fit.s.root[i][tid]);
+        nm = fgeom::fit7_models(basis, roots, nr, Fw);
+    }
     // the models' place in the list: prefix of nm in lane order (the lanes
     // past the samples add nothing)
     uint32_t inc = (uint32_t)nm;
@@ -499,7 +545,10 @@ __global__ __launch_bounds__(kS7Block, 4) void score7_kernel(const Src batch, fl
     }
 }
 
-// best 7-point hypothesis (largest count, lowest index), its best model and mask
+// best 7-point hypothesis (largest count, lowest index), and the mask of its best
+// model where one is asked for. The model is read if the scorer stored it; else
+// it is solved again and the sample's models recounted, which a caller that takes
+// no mask does not pay (32 pairs x 4096 samples: 50 -> 7 us).
 template <int kMode, class Src>
 __global__ __launch_bounds__(kThreads) void best7_kernel(const Src batch, float t2, float s0, float s1)
 {
@@ -523,36 +572,46 @@ __global__ __launch_bounds__(kThreads) void best7_kernel(const Src batch, float 
     const uint64_t bk = sKey[0];
     const uint32_t bestH = T.H ? ~(uint32_t)bk : 0u;
     const uint32_t bestC = (uint32_t)(bk >> 32);
+    if (threadIdx.x == 0 && T.best) {
+        T.best[0] = T.H ? bestH : ~0u;
+        T.best[1] = bestC;
+    }
+    if (!T.mask) return;
+    const bool found = T.H > 0 && bestC > 0;
     if (threadIdx.x == 0) {
         float Fs[kMaxF7][9];
-        const int nm = (T.H > 0 && bestC > 0) ? fit_hypothesis7(T, n, bestH, s0, s1, Fs) : 0;
+        float4 p[7];
+        int nm = 0;
+        if (found && T.models) {
+            for (int q = 0; q < 9; q++) Fs[0][q] = T.models[(size_t)bestH * 9 + q];
+            nm = 1;
+        } else if (found && load_sample7(T, n, bestH, s0, s1, p)) {
+            nm = fgeom::fit7(p, Fs);
+        }
         for (int m = 0; m < kMaxF7; m++)
             for (int q = 0; q < 9; q++) sFs[m][q] = m < nm ? Fs[m][q] : 0.f;
         sNm = nm;
     }
     __syncthreads();
     const int nm = sNm;
-    // counts of the (up to three) models of the best sample
-    uint32_t c[kMaxF7] = {0, 0, 0};
-    for (uint32_t i = threadIdx.x; i < n; i += kThreads) {
-        const float4 p = T.pts[i];
-        for (int m = 0; m < nm; m++) c[m] += fgeom::inlier<kMode>(sFs[m], p, t2) ? 1u : 0u;
-    }
-    for (int m = 0; m < kMaxF7; m++) sRed[m][threadIdx.x] = c[m];
-    __syncthreads();
-    for (int s = kThreads / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s)
-            for (int m = 0; m < kMaxF7; m++) sRed[m][threadIdx.x] += sRed[m][threadIdx.x + s];
-        __syncthreads();
-    }
     int bm = 0;
-    for (int m = 1; m < nm; m++)
-        if (sRed[m][0] > sRed[bm][0]) bm = m;
-    if (threadIdx.x == 0 && T.best) {
-        T.best[0] = T.H ? bestH : ~0u;
-        T.best[1] = bestC;
+    if (nm > 1) {
+        // counts of the two or three models of the best sample
+        uint32_t c[kMaxF7] = {0, 0, 0};
+        for (uint32_t i = threadIdx.x; i < n; i += kThreads) {
+            const float4 p = T.pts[i];
+            for (int m = 0; m < nm; m++) c[m] += fgeom::inlier<kMode>(sFs[m], p, t2) ? 1u : 0u;
+        }
+        for (int m = 0; m < kMaxF7; m++) sRed[m][threadIdx.x] = c[m];
+        __syncthreads();
+        for (int s = kThreads / 2; s > 0; s >>= 1) {
+            if (threadIdx.x < s)
+                for (int m = 0; m < kMaxF7; m++) sRed[m][threadIdx.x] += sRed[m][threadIdx.x + s];
+            __syncthreads();
+        }
+        for (int m = 1; m < nm; m++)
+            if (sRed[m][0] > sRed[bm][0]) bm = m;
     }
-    if (!T.mask) return;
     float F[9];
     for (int q = 0; q < 9; q++) F[q] = sFs[bm][q];
     for (uint32_t i = threadIdx.x; i < T.nHost; i += kThreads)
