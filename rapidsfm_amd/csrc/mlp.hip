@@ -359,7 +359,9 @@ __device__ inline v8bf row8(const __bf16* row, int k0) { return *reinterpret_cas
 //   12,13  layer 1: ob = blk - 12; B columns 0..7 = inputs, 8 = ones
 //   14..16 layer 4: ib = blk - 14, A row 0 = dz
 constexpr int kBlocks = 17;
-constexpr int kBlocksPerWave = (kBlocks + kWaves - 1) / kWaves;
+constexpr int kGradWaves = 8;  // wavefronts of the gradient kernel
+constexpr int kBlocksPerWave = (kBlocks + kGradWaves - 1) / kGradWaves;
+static_assert(kGradWaves >= kWaves && kGradWaves <= kBlocks, "every wave has a block");
 
 __device__ inline v16f grad_block_step(const Trans& T, int blk, int lane, v16f acc)
 {
@@ -423,9 +425,16 @@ __device__ inline void grad_block_store(float* __restrict__ out, int blk, int la
 
 // Per-workgroup partial gradient of the mean BCE over n samples (scale invN)
 // and partial loss sum: partials[wg][0 .. kNParam) and partials[wg][kNParam].
-__global__ __launch_bounds__(256) void grad_kernel(const float* __restrict__ P, const float* __restrict__ X,
-                                                   const float* __restrict__ Y, uint32_t n, float invN,
-                                                   float* __restrict__ partials)
+// A step's 128 matches go forward and back on the first four wavefronts, 32
+// each; all eight gather the operands and compute the 17 gradient blocks. LDS
+// holds one workgroup per CU, so waves that only help cost no other workgroup;
+// nine or more would leave 168 registers and spill 125 (eight: 256, 25 spilled,
+// with each layer stored before the next layer's product to keep them few).
+// Gradient and reduction over 8192 matches: four waves with up to five blocks
+// each 21.0 us, eight with up to three 18.8.
+__global__ __launch_bounds__(64 * kGradWaves) void grad_kernel(const float* __restrict__ P, const float* __restrict__ X,
+                                                               const float* __restrict__ Y, uint32_t n, float invN,
+                                                               float* __restrict__ partials)
 {
     __shared__ Ops S;
     __shared__ Trans T;
@@ -440,71 +449,76 @@ __global__ __launch_bounds__(256) void grad_kernel(const float* __restrict__ P, 
     float lossSum = 0.f;
 
     for (uint32_t stepBase = blockIdx.x * kStep; stepBase < n; stepBase += gridDim.x * kStep) {
-        const uint32_t base = stepBase + wave * 32;
-        Acts A;
-        const float z = forward_tile(S, X, n, base, lane, A);
-        const uint32_t idx = base + (lane & 31);
-        const bool valid = idx < n;
-        const float y = valid ? Y[idx] : 0.f;
-        const float p = 1.f / (1.f + __expf(-z));
-        const float dz = valid ? (p - y) * invN : 0.f;
-        if (valid && hi == 0) lossSum += fmaxf(z, 0.f) - y * z + log1pf(__expf(-fabsf(z)));
+        if (wave < kWaves) {
+            const uint32_t base = stepBase + wave * 32;
+            Acts A;
+            const float z = forward_tile(S, X, n, base, lane, A);
+            const uint32_t idx = base + (lane & 31);
+            const bool valid = idx < n;
+            const float y = valid ? Y[idx] : 0.f;
+            const float p = 1.f / (1.f + __expf(-z));
+            const float dz = valid ? (p - y) * invN : 0.f;
+            if (valid && hi == 0) lossSum += fmaxf(z, 0.f) - y * z + log1pf(__expf(-fabsf(z)));
 
-        // deltas: g3 = dz * W4 (masked by h3 > 0), then through W3^T and W2^T
-        v8bf g3[4], g2[4], g1[4];
+            // deltas: g3 = dz * W4 (masked by h3 > 0), then through W3^T and W2^T;
+            // each layer's are transposed into the step arrays before the next layer's product
+            v8bf g3[4], g2[4], g1[4];
 #pragma unroll
-        for (int t = 0; t < 4; t++)
+            for (int t = 0; t < 4; t++)
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float h = from_bf(A.h3[t][j]);
-                g3[t][j] = to_bf(h > 0.f ? dz * S.w4[hi][8 * t + j] : 0.f);
-            }
-        v16f c[2];
+                for (int j = 0; j < 8; j++) {
+                    const float h = from_bf(A.h3[t][j]);
+                    g3[t][j] = to_bf(h > 0.f ? dz * S.w4[hi][8 * t + j] : 0.f);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            store_packed(T.h3, A.h3, col, hi);
+            store_packed(T.g3, g3, col, hi);
+            v16f c[2];
 #pragma unroll
-        for (int rb = 0; rb < 2; rb++) {
-            v16f s = zero16();
+            for (int rb = 0; rb < 2; rb++) {
+                v16f s = zero16();
 #pragma unroll
-            for (int t = 0; t < 4; t++) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(S.w3t[rb][t][lane], g3[t], s, 0, 0, 0);
-            c[rb] = s;
-        }
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float h = from_bf(A.h2[t][j]);
-                g2[t][j] = to_bf(h > 0.f ? c[t >> 1][8 * (t & 1) + j] : 0.f);
+                for (int t = 0; t < 4; t++) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(S.w3t[rb][t][lane], g3[t], s, 0, 0, 0);
+                c[rb] = s;
             }
 #pragma unroll
-        for (int rb = 0; rb < 2; rb++) {
-            v16f s = zero16();
+            for (int t = 0; t < 4; t++)
 #pragma unroll
-            for (int t = 0; t < 4; t++) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(S.w2t[rb][t][lane], g2[t], s, 0, 0, 0);
-            c[rb] = s;
-        }
+                for (int j = 0; j < 8; j++) {
+                    const float h = from_bf(A.h2[t][j]);
+                    g2[t][j] = to_bf(h > 0.f ? c[t >> 1][8 * (t & 1) + j] : 0.f);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            store_packed(T.h2, A.h2, col, hi);
+            store_packed(T.g2, g2, col, hi);
 #pragma unroll
-        for (int t = 0; t < 4; t++)
+            for (int rb = 0; rb < 2; rb++) {
+                v16f s = zero16();
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float h = from_bf(A.h1[t][j]);
-                g1[t][j] = to_bf(h > 0.f ? c[t >> 1][8 * (t & 1) + j] : 0.f);
+                for (int t = 0; t < 4; t++) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(S.w2t[rb][t][lane], g2[t], s, 0, 0, 0);
+                c[rb] = s;
             }
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const float h = from_bf(A.h1[t][j]);
+                    g1[t][j] = to_bf(h > 0.f ? c[t >> 1][8 * (t & 1) + j] : 0.f);
+                }
 
-        // transpose this wave's 32 matches into the step arrays
-        store_packed(T.g3, g3, col, hi);
-        store_packed(T.h2, A.h2, col, hi);
-        store_packed(T.g2, g2, col, hi);
-        store_packed(T.h1, A.h1, col, hi);
-        store_packed(T.g1, g1, col, hi);
-        store_packed(T.h3, A.h3, col, hi);
-        if (hi == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            store_packed(T.g1, g1, col, hi);
+            store_packed(T.h1, A.h1, col, hi);
+            if (hi == 0) {
 #pragma unroll
-            for (int j = 0; j < 8; j++) T.x[j][col] = A.x[j];
-            T.dz[col] = to_bf(dz);
+                for (int j = 0; j < 8; j++) T.x[j][col] = A.x[j];
+                T.dz[col] = to_bf(dz);
+            }
         }
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < kBlocksPerWave; j++) {
-            const int blk = wave + kWaves * j;
+            const int blk = wave + kGradWaves * j;
             if (blk < kBlocks) acc[j] = grad_block_step(T, blk, lane, acc[j]);
         }
         __syncthreads();
@@ -513,12 +527,12 @@ __global__ __launch_bounds__(256) void grad_kernel(const float* __restrict__ P, 
     float* out = partials + (size_t)blockIdx.x * (kNParam + 1);
 #pragma unroll
     for (int j = 0; j < kBlocksPerWave; j++) {
-        const int blk = wave + kWaves * j;
+        const int blk = wave + kGradWaves * j;
         if (blk < kBlocks) grad_block_store(out, blk, lane, acc[j]);
     }
     // loss: wave sum, then workgroup sum
     for (int o = 32; o > 0; o >>= 1) lossSum += __shfl_xor(lossSum, o);
-    if (lane == 0) T.loss[wave] = lossSum;
+    if (lane == 0 && wave < kWaves) T.loss[wave] = lossSum;
     __syncthreads();
     if (threadIdx.x == 0) {
         float s = 0.f;
@@ -628,9 +642,14 @@ __global__ void features_kernel(const FeatBatch batch)
 
 static uint32_t grad_grid(uint32_t n)
 {
-    // enough workgroups to fill the chip, at least one step each
-    return std::max(1u, std::min<uint32_t>(512u, div_up(n, kStep)));
+    // at least one step each, and a workgroup per CU, as many as its LDS lets run:
+    // twice as many gathered the operands and wrote their partials twice (gradient
+    // and reduction over 65536 matches, 512 workgroups 46 us, 256 34 us)
+    return std::max(1u, std::min<uint32_t>(256u, div_up(n, kStep)));
 }
+
+// partials a workspace must hold; kept above the grid, callers size theirs by it
+static uint32_t grad_partials(uint32_t n) { return std::max(1u, std::min<uint32_t>(512u, div_up(n, kStep))); }
 
 }  // namespace mlp
 }  // namespace rsfm_amd
@@ -653,7 +672,7 @@ extern "C" int rsfm_mlp_forward(const float* params, const float* x, uint32_t n,
 extern "C" int rsfm_mlp_grad_workspace_size(uint32_t n, size_t* bytes)
 {
     RSFM_RETURN_IF(bytes == nullptr, RSFM_ERR_INVALID, "bytes is null");
-    *bytes = (size_t)mlp::grad_grid(n) * (mlp::kNParam + 1) * sizeof(float);
+    *bytes = (size_t)mlp::grad_partials(n) * (mlp::kNParam + 1) * sizeof(float);
     return RSFM_OK;
 }
 
@@ -670,7 +689,7 @@ extern "C" int rsfm_mlp_grad(const float* params, const float* x, const float* y
                    "mlp grad: workspace too small (" + std::to_string(workspaceBytes) + " < " + std::to_string(need) + ")");
     const uint32_t grid = mlp::grad_grid(n);
     float* part = static_cast<float*>(workspace);
-    mlp::grad_kernel<<<grid, 256, 0, stream>>>(params, x, y, n, 1.f / (float)n, part);
+    mlp::grad_kernel<<<grid, 64 * mlp::kGradWaves, 0, stream>>>(params, x, y, n, 1.f / (float)n, part);
     RSFM_CHECK(check_launch("mlp grad"));
     mlp::reduce_kernel<<<div_up(mlp::kNParam + 1, mlp::kRedParams), mlp::kRedParams * mlp::kRedGroups, 0, stream>>>(part, grid, n, grad, loss);
     return check_launch("mlp grad reduce");

@@ -51,8 +51,9 @@ def test_forward_not_a_number(dev):
     assert torch.equal(out[keep], clean[keep])
 
 
-# partial counts around the reduction's eight groups of eight: 1, 7, 8, 9, 63, 64, 65 and 512 workgroups
-@pytest.mark.parametrize("n", [100, 896, 1024, 1152, 8064, 8192, 8320, 70000])
+# partial counts around the reduction's eight groups of eight: 1, 7, 8, 9, 63, 64, 65 workgroups; all 256
+# with a step each, one match more, and several ragged steps
+@pytest.mark.parametrize("n", [100, 896, 1024, 1152, 8064, 8192, 8320, 32768, 32769, 70000])
 def test_gradient_sum_edges(dev, n):
     from rapidsfm_amd import learned as L
 
