@@ -34,16 +34,22 @@ def _ptr(t):
     return t.data_ptr() if t is not None and t.numel() > 0 else 0
 
 
-def _rows(likes, counts, cols, dtype):
+def _rows(likes, counts, cols, dtype, align=256):
     """One tensor per count, (count, cols) or (count,) for cols None, each on the device of
     its entry of likes. The parts of a batch on one device are cut from one allocation, from
-    row numbers that are multiples of 256 so that each stays aligned: a dozen allocations
+    row numbers that are multiples of align so that each stays aligned: a dozen allocations
     cost the host more than the launches they are for."""
     shape = (lambda n: (n,)) if cols is None else (lambda n: (n, cols))  # noqa: E731
     if len(counts) < 2 or any(t.device != likes[0].device for t in likes):
         return [torch.empty(shape(n), dtype=dtype, device=t.device) for t, n in zip(likes, counts)]
-    sizes = [m for n in counts for m in (n, -n % 256)]
-    return torch.empty(shape(sum(sizes)), dtype=dtype, device=likes[0].device).split(sizes)[::2]
+    sizes, at = [], []
+    for n in counts:
+        at.append(len(sizes))
+        sizes.append(n)
+        if n % align:
+            sizes.append(-n % align)
+    parts = torch.empty(shape(sum(sizes)), dtype=dtype, device=likes[0].device).split(sizes)
+    return [parts[i] for i in at]
 
 
 def _check_desc(d, width=128):
@@ -308,7 +314,7 @@ def _ransac_tasks(problems, want_models):
             raise ValueError("pts must be contiguous float32 (n, 4)")
     ns, hs = [t.shape[0] for t in likes], [prob[1].shape[0] for prob in problems]
     counts, masks = _rows(likes, hs, None, torch.int32), _rows(likes, ns, None, torch.uint8)
-    bests = _rows(likes, [2] * len(likes), None, torch.int32)
+    bests = _rows(likes, [2] * len(likes), None, torch.int32, align=2)
     models = [None] * len(likes)
     if want_models:
         models = [m.view(h, 3, 3) for m, h in zip(_rows(likes, hs, 9, torch.float32), hs)]

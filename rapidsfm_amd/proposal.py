@@ -159,7 +159,7 @@ def score(problems, threshold=1.0):
     likes = [pts for pts, _ in problems]
     counts = _rows(likes, [idx.shape[0] for _, idx in problems], None, torch.int32)
     masks = _rows(likes, [max(1, t.shape[0]) for t in likes], None, torch.uint8)
-    bests = _rows(likes, [2] * len(likes), None, torch.int32)
+    bests = _rows(likes, [2] * len(likes), None, torch.int32, align=2)
     arr = (RansacTask * max(1, len(problems)))()
     outs = []
     for i, (pts, idx) in enumerate(problems):
