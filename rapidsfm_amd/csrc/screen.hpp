@@ -267,23 +267,26 @@ __device__ inline Coef make_coef(const Box& B, const float F[9], bool ok, float 
     const double sk = inRange ? pow2d(k) : 0.0, sq = inRange ? pow2d(2 * k) : 0.0;
     // out of range: every test of the model stays open
     const bool open = !inRange || !(c * sq < 1e20) || !(de * sk < 1e15);
-    const double fe = ok && !open ? sk : 0.0, fq = ok && !open ? sq * kOne : 0.0;
+    const bool use = ok && !open;
+    // chosen, not multiplied by zero: out of range they may be infinite or NaN
+    auto coef = [&](double x, double f) { return use ? (float)(x * f) : 0.f; };
+    const double fq = sq * kOne;
 #pragma unroll
-    for (int i = 0; i < 9; i++) r.e[i] = (float)(G[i / 3][i % 3] * fe);
+    for (int i = 0; i < 9; i++) r.e[i] = coef(G[i / 3][i % 3], sk);
 #pragma unroll
     for (int m = 0; m < 2; m++)
 #pragma unroll
-        for (int i = 0; i < 5; i++) r.q[m][i] = (float)(Q[m][i] * fq);
+        for (int i = 0; i < 5; i++) r.q[m][i] = coef(Q[m][i], fq);
     if (kMode == 1) {
-        r.k[0] = (float)((Q[0][5] + Q[1][5]) * fq);
+        r.k[0] = coef(Q[0][5] + Q[1][5], fq);
         r.k[1] = 0.f;
     } else {
-        r.k[0] = (float)(Q[0][5] * fq);
-        r.k[1] = (float)(Q[1][5] * fq);
+        r.k[0] = coef(Q[0][5], fq);
+        r.k[1] = coef(Q[1][5], fq);
     }
     // an open model has e = D = 0, so g = 0; kFar^2 kOne^2 of a padding point exceeds every c
-    r.d2 = ok && !open ? (float)(2.02 * de * sk * kOne) : 0.f;
-    r.c = ok && !open ? (float)(c * sq * kOne * kOne) : 1.f;
+    r.d2 = use ? (float)(2.02 * de * sk * kOne) : 0.f;
+    r.c = use ? (float)(c * sq * kOne * kOne) : 1.f;
     return r;
 }
 

@@ -83,3 +83,28 @@ def test_beyond_the_bound(orc, dev, kind, mode, what):
     else:
         t = 1e-9 if what == "tiny_t" else 1e12
     _check(orc, dev, pts, 130, mode, t, 3, kind)
+
+
+# "no limit" as the threshold: its square is infinite in FP32, every point with a
+# finite distance is an inlier; point counts that leave padding in the last tile
+@pytest.mark.parametrize("kind", ["f8", "f7"])
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("n", [15, 181])
+@pytest.mark.parametrize("t", [float("inf"), 2e19])
+def test_no_limit(orc, dev, kind, mode, n, t):
+    pts, _, _, _ = plane_scene(10, n // 3, n // 3, n - 2 * (n // 3), noise=0.5)
+    _check(orc, dev, pts, 130, mode, t, 5, kind)
+
+
+# the same on the 256-hypothesis workgroups
+@pytest.mark.parametrize("mode", [0, 1])
+def test_no_limit_wide(orc, dev, mode):
+    from rapidsfm_amd import ops
+
+    print("[case] screen wide, no limit", mode, flush=True)
+    pts, _, _, _ = plane_scene(6, 40, 40, 37, noise=0.5)
+    idx = [_idx(117, 1024, 8, 60 + k) for k in range(32)]
+    outs = ops.ransac_f8([(_dev(pts, dev), _dev(i, dev)) for i in idx], float("inf"), mode=mode)
+    for i, o in zip(idx, outs):
+        c, _ = orc.f8_score(pts, i, float("inf"), mode, nthreads=8)
+        assert np.array_equal(o["counts"].cpu().numpy().view(np.uint32), c)
