@@ -254,8 +254,12 @@ __device__ __forceinline__ uint32_t count_inliers(CountSmem& S, const Cells& c, 
                      6.2e-5f * (t3 + t4 + 3.f) + 1e-6f * (f.x + f.y);
     const float cc = 1.05f * (2.f * th * (e0 + e1) + e0 * e0 + e1 * e1 + 16.f * u * sq);
     // a model that maps the whole neighbourhood further from its matches than the
-    // threshold (another cell's, extrapolated) has no inlier; the margins cover e0, e1
-    if (a0 * 0.9999f > t0 * f.x + t1 * f.y + f.z + 2.f * th || a1 * 0.9999f > t3 * f.x + t4 * f.y + f.w + 2.f * th) live = false;
+    // threshold (another cell's, extrapolated) has no inlier: in exact arithmetic
+    // d0 is at least a0 - (t0 x + t1 y + z) throughout, and e0 holds the FP32
+    // expression's own roundings, which for a steep model exceed the threshold;
+    // the second th and e0 and the 1e-4 are for the roundings of these lines
+    if (a0 * 0.9999f > t0 * f.x + t1 * f.y + f.z + 2.f * (th + e0) || a1 * 0.9999f > t3 * f.x + t4 * f.y + f.w + 2.f * (th + e1))
+        live = false;
     // beyond f16's range: every test of the model is open
     const bool open = live && !(fmaxf(fmaxf(t0, t1), fmaxf(t3, t4)) < 500.f && fmaxf(a0, a1) < 30000.f && sq < 1e8f && cc < 1e8f);
     const bool use = live && !open;

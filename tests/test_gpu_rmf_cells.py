@@ -74,3 +74,32 @@ def test_cell_counts(orc, dev, cell_cols):
     m = _matches(6, 1500, 900.0, 10.0)
     m[::2, :2] = rng.uniform([0, 0], [4000, 3000], (750, 2))
     _check(orc, dev, m, cell_cols, 128, 0.15, True, 1)
+
+
+# A steep affine (area kept, one axis stretched T0 times) of one cell, tried on a
+# far cell whose matches it hits exactly in FP32: the expression's own rounding
+# there, the larger the steeper, is beyond the threshold, and the test accepts
+# what the affine in exact arithmetic misses by more than twice the threshold.
+@pytest.mark.parametrize("t0,th", [(250.0, 0.005), (400.0, 0.02), (2001.0, 0.1), (30000.0, 1.0)])
+@pytest.mark.parametrize("n", [16, 40])
+def test_steep_affine_of_another_cell(orc, dev, t0, th, n):
+    print("[case] rmf steep", t0, th, n, flush=True)
+    rng = np.random.default_rng(1)
+    left = np.stack([rng.uniform(2990, 3010, 40), rng.uniform(2400, 2600, 40)], 1).astype(np.float32)
+    right = np.stack([(left[:, 0].astype(np.float64) - 3000) * t0 + 2000, (left[:, 1] - 2500.0) / t0 + 1500], 1)
+    steep = np.concatenate([left, right], 1).astype(np.float32)
+    rel, seed = th / 250, 7
+    r, bounds, _, cols, rows, cw = orc.rmf_bin(4000, 3000, steep, 16)
+    assert cw == 250
+    _, aff = orc.rmf_filter(r, bounds, cols, rows, 256, cw * rel, True, seed)
+    T = aff[10 * cols + 12]
+    assert abs(T[0] - t0) < 0.01 * t0
+    # of the x near 3000 the one where FP32 is furthest from exact arithmetic
+    xs = np.unique(rng.uniform(2995, 3005, 4000).astype(np.float32))
+    y = np.float32(500.25)
+    fl = ((T[0] * xs + T[1] * y) + T[2]).astype(np.float32)
+    off = np.abs(T[0].astype(np.float64) * xs + T[1].astype(np.float64) * y + T[2] - fl)
+    k = int(np.argmax(off))
+    assert off[k] > 2.2 * th
+    hit = np.array([xs[k], y, fl[k], (T[3] * xs[k] + T[4] * y) + T[5]], np.float32)
+    _check(orc, dev, np.concatenate([steep, np.tile(hit, (n, 1))]), 16, 256, rel, True, seed)
