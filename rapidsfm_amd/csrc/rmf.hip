@@ -123,19 +123,27 @@ struct Frame {
     bool odd;  // coordinates beyond the bound: every test is exact
 };
 
-__device__ inline float wave_max(float x)
+// largest value of the wave (float or uint32_t)
+template <class V>
+__device__ inline V wave_max(V x)
 {
-    const auto dpp = [](float v, auto k) {
-        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(k)::value, 0xF, 0xF, true));
+    const auto most = [](V a, V b) {
+        if constexpr (std::is_same_v<V, float>) return fmaxf(a, b);
+        else return max(a, b);
     };
-    x = fmaxf(x, dpp(x, std::integral_constant<int, 0xB1>{}));   // quad_perm: neighbour
-    x = fmaxf(x, dpp(x, std::integral_constant<int, 0x4E>{}));   // quad_perm: other pair
-    x = fmaxf(x, dpp(x, std::integral_constant<int, 0x141>{}));  // row_half_mirror
-    x = fmaxf(x, dpp(x, std::integral_constant<int, 0x140>{}));  // row_mirror
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    const auto dpp = [](V v, auto k) {
+        return __builtin_bit_cast(V, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(k)::value, 0xF, 0xF, true));
+    };
+    x = most(x, dpp(x, std::integral_constant<int, 0xB1>{}));   // quad_perm: neighbour
+    x = most(x, dpp(x, std::integral_constant<int, 0x4E>{}));   // quad_perm: other pair
+    x = most(x, dpp(x, std::integral_constant<int, 0x141>{}));  // row_half_mirror
+    x = most(x, dpp(x, std::integral_constant<int, 0x140>{}));  // row_mirror
+    uint32_t u = __builtin_bit_cast(uint32_t, x);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    x = most(__builtin_bit_cast(V, (uint32_t)a[0]), __builtin_bit_cast(V, (uint32_t)a[1]));
+    u = __builtin_bit_cast(uint32_t, x);
+    const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return most(__builtin_bit_cast(V, (uint32_t)b[0]), __builtin_bit_cast(V, (uint32_t)b[1]));
 }
 
 __device__ inline void frame_add(Frame& f, const float4& p)
@@ -416,30 +424,32 @@ __device__ inline uint32_t lcg(uint32_t& s)
 }
 
 struct Reducer {
-    uint32_t key[kCta / 64];
+    uint32_t cnt[kCta / 64], order[kCta / 64];
     float aff[6];
 };
 
 // CtaReducer::findMax: the largest count; among equals its tree (thread t keeps
 // its value unless t + mid holds a strictly larger count, mid = 64 .. 1) leaves
 // the thread whose reversed index is lowest. The winner's count and affine are
-// returned to every thread.
+// returned to every thread. Count and order are reduced one after the other: a
+// key of both in 32 bits would leave the count 25.
 __device__ __forceinline__ void cta_find_max(Reducer& R, uint32_t& cnt, float T[6])
 {
-    static_assert(kCta == 128, "seven index bits");
-    const uint32_t order = 127u - (__brev(threadIdx.x) >> 25);
-    const uint32_t mine = (cnt << 7) | order;  // fewer than 2^25 matches in a neighbourhood
-    uint32_t key = mine;
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) key = max(key, (uint32_t)__shfl_xor((int)key, s));
-    if ((threadIdx.x & 63) == 0) R.key[threadIdx.x >> 6] = key;
+    static_assert(kCta == 128, "seven index bits, two waves");
+    const uint32_t mine = 128u - (__brev(threadIdx.x) >> 25);
+    const uint32_t most = wave_max(cnt), first = wave_max(cnt == most ? mine : 0u);
+    if ((threadIdx.x & 63) == 0) {
+        R.cnt[threadIdx.x >> 6] = most;
+        R.order[threadIdx.x >> 6] = first;
+    }
     __syncthreads();
-    key = max(R.key[0], R.key[1]);
-    if (mine == key)
+    const uint32_t c0 = R.cnt[0], c1 = R.cnt[1], o0 = R.order[0], o1 = R.order[1];
+    const bool second = c1 > c0 || (c1 == c0 && o1 > o0);
+    if (mine == (second ? o1 : o0))
 #pragma unroll
         for (int q = 0; q < 6; q++) R.aff[q] = T[q];
     __syncthreads();
-    cnt = key >> 7;
+    cnt = second ? c1 : c0;
 #pragma unroll
     for (int q = 0; q < 6; q++) T[q] = R.aff[q];
 }

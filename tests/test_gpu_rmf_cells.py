@@ -103,3 +103,16 @@ def test_steep_affine_of_another_cell(orc, dev, t0, th, n):
     assert off[k] > 2.2 * th
     hit = np.array([xs[k], y, fl[k], (T[3] * xs[k] + T[4] * y) + T[5]], np.float32)
     _check(orc, dev, np.concatenate([steep, np.tile(hit, (n, 1))]), 16, 256, rel, True, seed)
+
+
+# more matches in one neighbourhood than 25 bits count
+def test_largest_neighbourhood(dev):
+    from rapidsfm_amd import rmf
+
+    n = (1 << 25) + 3
+    print("[case] rmf neighbourhood", n, flush=True)
+    g = torch.Generator(device=dev).manual_seed(1)
+    m = torch.rand((n, 2), generator=g, device=dev) * 3000.0
+    votes, _ = rmf.filter_votes(torch.cat([m, m], 1), torch.tensor([0, n], dtype=torch.int32, device=dev), 1, 1, 128,
+                                8.0, False, 3)
+    assert int((votes == 1).sum()) == n
