@@ -104,7 +104,8 @@ class Adam:
 
 
 def sample_weighted(tasks, stream=None):
-    """tasks: list of (weights float32 (n,), H, seed[, n_dev int32 (1,)]) -> list of (H, 8) int32 index sets."""
+    """tasks: list of (weights float32 (n,), H, seed[, n_dev int32 (1,)]) -> list of (H, 8) int32 index sets,
+    which share one allocation (clone() one that is to outlive the rest, be saved alone or be resized)."""
     arr = (WSampleTask * max(1, len(tasks)))()
     likes = [t[0] for t in tasks]
     outs = _rows(likes, [t[1] for t in tasks], 8, torch.int32)

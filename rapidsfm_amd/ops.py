@@ -35,11 +35,14 @@ def _ptr(t):
 
 
 def _rows(likes, counts, cols, dtype, align=256):
-    """One tensor per count, (count, cols) or (count,) for cols None, each on the device of
+    """One tensor per count, (count, cols...) or (count,) for cols None, each on the device of
     its entry of likes. The parts of a batch on one device are cut from one allocation, from
     row numbers that are multiples of align so that each stays aligned: a dozen allocations
-    cost the host more than the launches they are for."""
-    shape = (lambda n: (n,)) if cols is None else (lambda n: (n, cols))  # noqa: E731
+    cost the host more than the launches they are for. They share that storage, which lives
+    as long as any of them, and nothing else: to autograd each is a tensor of its own, no view,
+    with its own version counter (unsafe_split; split gives views of one another's base)."""
+    tail = () if cols is None else (cols if isinstance(cols, tuple) else (cols,))
+    shape = lambda n: (n,) + tail  # noqa: E731
     if len(counts) < 2 or any(t.device != likes[0].device for t in likes):
         return [torch.empty(shape(n), dtype=dtype, device=t.device) for t, n in zip(likes, counts)]
     sizes, at = [], []
@@ -48,7 +51,8 @@ def _rows(likes, counts, cols, dtype, align=256):
         sizes.append(n)
         if n % align:
             sizes.append(-n % align)
-    parts = torch.empty(shape(sum(sizes)), dtype=dtype, device=likes[0].device).split(sizes)
+    parts = torch.empty(shape(sum(sizes)), dtype=dtype, device=likes[0].device)
+    parts = torch.unsafe_split_with_sizes(parts, sizes)
     return [parts[i] for i in at]
 
 
@@ -136,7 +140,7 @@ def bf_match_top2(pairs, stream=None, workspace=None):
 
 def ransac_f7(problems, threshold, mode=1, min_sep_sq=(0.0, 0.0), want_models=False, stream=None):
     """7-point hypotheses: like ransac_f8 with sampleIdx of shape (H, 7); each
-    hypothesis reports its best of up to three F."""
+    hypothesis reports its best of up to three F. Outputs share storage as ransac_f8's do."""
     return _ransac(lib.rsfm_ransac_f7, "rsfm_ransac_f7", problems, threshold, mode, min_sep_sq, want_models, stream)
 
 
@@ -259,7 +263,8 @@ def pose_from_h(problems, front_ratio=0.95, stream=None):
 
 def ransac_h4(problems, threshold, min_sep_sq=(0.0, 0.0), want_models=False, stream=None):
     """4-point homography hypotheses: problems of (pts, sampleIdx (H, 4)[, nDev]);
-    the inlier test is checkProjectiveTransformation's with threshold t pixels."""
+    the inlier test is checkProjectiveTransformation's with threshold t pixels. Outputs
+    share storage as ransac_f8's do."""
     tasks, outs = _ransac_tasks(problems, want_models)
     check(lib.rsfm_ransac_h4(tasks, len(problems), float(threshold),
                              float(min_sep_sq[0]), float(min_sep_sq[1]), _stream(stream)), "rsfm_ransac_h4")
@@ -272,7 +277,9 @@ def ransac_f8(problems, threshold, mode=1, min_sep_sq=(0.0, 0.0), want_models=Fa
     pts: float32 CUDA (n, 4) [x0, y0, x1, y1]; sampleIdx: int32/uint32 CUDA (H, 8);
     nDev: optional int32 CUDA (1,) count. mode 0 = reference two-sided line test,
     1 = Sampson. Returns a list of dicts with counts (H,), best (2,), mask (n,) and
-    models (H, 3, 3) when asked.
+    models (H, 3, 3) when asked. The outputs of one kind share one allocation over
+    the problems: keep a clone() of those that are to outlive the rest, be saved
+    alone or be resized.
     """
     return _ransac(lib.rsfm_ransac_f8, "rsfm_ransac_f8", problems, threshold, mode, min_sep_sq, want_models, stream)
 
@@ -315,9 +322,7 @@ def _ransac_tasks(problems, want_models):
     ns, hs = [t.shape[0] for t in likes], [prob[1].shape[0] for prob in problems]
     counts, masks = _rows(likes, hs, None, torch.int32), _rows(likes, ns, None, torch.uint8)
     bests = _rows(likes, [2] * len(likes), None, torch.int32, align=2)
-    models = [None] * len(likes)
-    if want_models:
-        models = [m.view(h, 3, 3) for m, h in zip(_rows(likes, hs, 9, torch.float32), hs)]
+    models = _rows(likes, hs, (3, 3), torch.float32) if want_models else [None] * len(likes)
     outs = []
     for i, prob in enumerate(problems):
         o = {"counts": counts[i], "best": bests[i], "mask": masks[i], "models": models[i]}

@@ -1,4 +1,4 @@
-"""The outputs of a batched call are parts of one allocation: each with its own rows,
+"""The outputs of a batched call are parts of one allocation: each with its own rows and version,
 aligned, for every count including none and one, on the device of its own problem."""
 import pytest
 import torch
@@ -23,3 +23,26 @@ def test_parts_are_disjoint_and_aligned(counts, cols, dtype):
 def test_parts_follow_their_problem_s_device():
     parts = ops._rows([torch.empty(1), torch.empty(1, device="meta")], [3, 4], None, torch.int32)
     assert [t.device.type for t in parts] == ["cpu", "meta"]
+
+
+def test_parts_are_tensors_of_their_own():
+    """what a caller can do with separate allocations: write in place under autograd, and write
+    one part while another is saved for a backward pass"""
+    a, b = ops._rows([torch.empty(1)] * 2, [3, 4], 9, torch.float32)
+    for t in (a, b):
+        assert not t._is_view() and not t.requires_grad
+        t.fill_(2.0)
+    w = torch.ones(3, 9, requires_grad=True)
+    y = (w * a).sum()  # saves a
+    b.zero_()
+    y.backward()
+    assert bool((w.grad == 2.0).all())
+    a.mul_(w)
+    assert a.requires_grad and not b.requires_grad
+
+
+def test_models_are_tensors_of_their_own():
+    pts = torch.zeros(20, 4)
+    idx = torch.zeros((5, 8), dtype=torch.int32)
+    _, outs = ops._ransac_tasks([(pts, idx), (pts, idx)], True)
+    assert all(o["models"].shape == (5, 3, 3) and not t._is_view() for o in outs for t in o.values())
