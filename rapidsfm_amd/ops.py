@@ -11,10 +11,16 @@ import torch
 from ._abi import BfTask, BfTop2Task, Camera, DegensacTask, FinishTask, PoseHTask, PoseTask, RansacTask, RealCamera, UndistortTask, check, lib
 
 
+# not part of torch's public interface, hence looked up: absent, the public way is taken
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(stream):
     """Raw stream handle; the current stream's without building a Stream object for it."""
     if stream is None:
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        if _current_raw_stream is None:
+            return torch.cuda.current_stream().cuda_stream
+        return _current_raw_stream(torch.cuda.current_device())
     return stream.cuda_stream
 
 

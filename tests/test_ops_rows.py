@@ -1,4 +1,4 @@
-"""The outputs of a batched call are parts of one allocation: each with its own rows and version,
+"""Host helpers. The outputs of a batched call are parts of one allocation: each with its own rows and version,
 aligned, for every count including none and one, on the device of its own problem."""
 import pytest
 import torch
@@ -46,3 +46,13 @@ def test_models_are_tensors_of_their_own():
     idx = torch.zeros((5, 8), dtype=torch.int32)
     _, outs = ops._ransac_tasks([(pts, idx), (pts, idx)], True)
     assert all(o["models"].shape == (5, 3, 3) and not t._is_view() for o in outs for t in o.values())
+
+
+def test_current_stream_without_the_private_call(monkeypatch):
+    class Stream:
+        cuda_stream = 42
+
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Stream)
+    monkeypatch.setattr(ops, "_current_raw_stream", None, raising=False)
+    assert ops._stream(None) == 42 and ops._stream(Stream) == 42
