@@ -86,6 +86,7 @@ def build(verbose=False, out=None):
         print("built", lib)
     if out is None:
         build_cpp_tests(verbose)
+        build_hip_tests(verbose)
     return lib
 
 
@@ -105,6 +106,21 @@ def build_cpp_tests(verbose=False):
     if verbose:
         print("built", exe)
     return exe
+
+
+def build_hip_tests(verbose=False):
+    """The GPU test's kernel for the matrix unit's sums (tests/hip/libmfma_sums.so)."""
+    src = os.path.join(ROOT, "tests", "hip", "mfma_sums.hip")
+    if not os.path.exists(src):
+        return None
+    lib = os.path.join(ROOT, "tests", "hip", "libmfma_sums.so")
+    cmd = [HIPCC, "-x", "hip"] + COMMON + DEVICE + ["-shared", src, "-o", lib]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("GPU test kernel failed to build: %s\n%s" % (" ".join(cmd), r.stderr))
+    if verbose:
+        print("built", lib)
+    return lib
 
 
 if __name__ == "__main__":

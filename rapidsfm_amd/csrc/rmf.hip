@@ -87,7 +87,7 @@ __device__ inline bool is_inlier(const float T[6], float4 p, float sq)
 // The bound, u = 2^-24, M = the largest magnitudes in the neighbourhood about
 // its first match, m the same in pixels: a staged term is off by 13 u (the
 // subtraction, two splits of 2^-22, the dropped lo * lo), the matrix unit's
-// FP32 sum by 10 u of the terms' magnitudes (5.4 u measured), halves below
+// FP32 sum by 10 u of the terms' magnitudes (assumed; 5.9 u measured), halves below
 // f16's normal range by 2^-14 absolute; the exact expression rounds at most
 // 3 u (|T0| mx + |T1| my) + 2 u (|T2| + mx').
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
