@@ -648,9 +648,6 @@ static uint32_t grad_grid(uint32_t n)
     return std::max(1u, std::min<uint32_t>(256u, div_up(n, kStep)));
 }
 
-// partials a workspace must hold; kept above the grid, callers size theirs by it
-static uint32_t grad_partials(uint32_t n) { return std::max(1u, std::min<uint32_t>(512u, div_up(n, kStep))); }
-
 }  // namespace mlp
 }  // namespace rsfm_amd
 
@@ -672,7 +669,7 @@ extern "C" int rsfm_mlp_forward(const float* params, const float* x, uint32_t n,
 extern "C" int rsfm_mlp_grad_workspace_size(uint32_t n, size_t* bytes)
 {
     RSFM_RETURN_IF(bytes == nullptr, RSFM_ERR_INVALID, "bytes is null");
-    *bytes = (size_t)mlp::grad_partials(n) * (mlp::kNParam + 1) * sizeof(float);
+    *bytes = (size_t)mlp::grad_grid(n) * (mlp::kNParam + 1) * sizeof(float);
     return RSFM_OK;
 }
 

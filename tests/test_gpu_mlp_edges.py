@@ -74,3 +74,30 @@ def test_gradient_sum_edges(dev, n):
     # the pieces round dz = (p - y) / m to bf16 at another scale: 2^-8 per product; the sums are FP32
     assert float((whole.double() - acc).norm() / acc.norm()) < 2.0**-8
     assert abs(float(loss) - lacc) < 1e-5 * max(1.0, abs(lacc))
+
+
+# a partial a workgroup is all that a gradient writes: the size asked for, up to the 256
+# workgroups' and no further, and nothing past it
+@pytest.mark.parametrize("n,partials", [(1, 1), (129, 2), (32768, 256), (32769, 256), (65537, 256)])
+def test_gradient_workspace(dev, n, partials):
+    import ctypes
+
+    from rapidsfm_amd import learned as L
+    from rapidsfm_amd._abi import lib
+
+    print("[case] mlp grad workspace", n, flush=True)
+    need = ctypes.c_size_t(0)
+    assert lib.rsfm_mlp_grad_workspace_size(n, ctypes.byref(need)) == 0
+    assert need.value == partials * (L.N_PARAM + 1) * 4
+    p = L.init_params(6, device=dev)
+    x = torch.randn((n, 8), device=dev)
+    y = (torch.rand(n, device=dev) < 0.4).float()
+    ws = torch.full((need.value // 4 + 4096,), 7.0, device=dev)
+    g, loss = torch.empty(L.N_PARAM, device=dev), torch.empty(1, device=dev)
+    call = lambda b: lib.rsfm_mlp_grad(p.data_ptr(), x.data_ptr(), y.data_ptr(), n, g.data_ptr(), loss.data_ptr(),  # noqa: E731
+                                       ws.data_ptr(), b, torch.cuda.current_stream().cuda_stream)
+    assert call(need.value - 1) != 0  # refused before any launch
+    assert call(need.value) == 0
+    rg, rl = L.grad(p, x, y)
+    assert torch.equal(g, rg) and torch.equal(loss, rl)
+    assert bool((ws[need.value // 4:] == 7.0).all())
