@@ -165,7 +165,7 @@ __device__ inline void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 //    the end of the tile the exact distances of the candidate (column, wave)
 //    pairs on MFMA, merged into bestB by atomicMin.
 template <int kBits, bool kTop2>
-__device__ __forceinline__ void match_tile_top2(const DevTask& T, uint32_t rowBase, uint32_t colBeg, uint32_t seg)
+__device__ __forceinline__ void match_tile_top2(const DevTask& T, uint32_t rowBase, uint32_t colBeg)
 {
     constexpr int kWaves = 8;
     constexpr int kChunkBytes = kBN * 128;
@@ -542,7 +542,7 @@ __global__ __launch_bounds__(512, 4) void match_top1_kernel(const Src batch)
     const uint32_t rowBase = wg.x * kBM;
     const uint32_t colBeg = wg.y * T.segCols;
     if (rowBase >= T.nA || colBeg >= T.nB) return;
-    match_tile_top2<kBits, false>(T, rowBase, colBeg, wg.y);
+    match_tile_top2<kBits, false>(T, rowBase, colBeg);
 }
 
 template <class Src>
@@ -553,7 +553,7 @@ __global__ __launch_bounds__(512, 4) void match_top2_kernel(const Src batch)
     const uint32_t rowBase = wg.x * kBM;
     const uint32_t colBeg = wg.y * T.segCols;
     if (rowBase >= T.nA || colBeg >= T.nB) return;
-    match_tile_top2<8, true>(T, rowBase, colBeg, wg.y);
+    match_tile_top2<8, true>(T, rowBase, colBeg);
 }
 
 // Persistent launch over a tile table: the tiles are split into kNumXcd lists
@@ -571,7 +571,7 @@ __global__ __launch_bounds__(512, 4) void match_tiles_kernel(const DevTask* __re
         const TileDesc d = tiles[i];
         const DevTask T = tasks[d.task];
         __syncthreads();  // the previous tile's last LDS reads
-        match_tile_top2<8, true>(T, d.rowBase, d.colBeg, d.seg);
+        match_tile_top2<8, true>(T, d.rowBase, d.colBeg);
     }
 }
 
@@ -587,7 +587,7 @@ __global__ __launch_bounds__(512, 4) void match_tile_grid_kernel(const DevTask* 
     if (i >= xcdOff[xcd + 1]) return;
     const TileDesc d = tiles[i];
     const DevTask T = tasks[d.task];
-    match_tile_top2<8, true>(T, d.rowBase, d.colBeg, d.seg);
+    match_tile_top2<8, true>(T, d.rowBase, d.colBeg);
 }
 
 // staging form of B (DevTask::W, NB): eight lanes per column, one 16-B slot

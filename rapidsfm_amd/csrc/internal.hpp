@@ -48,7 +48,7 @@ typedef InTable<DevTask> TaskTable;
 
 // one workgroup tile of the batched pipeline: kBM query rows x one segment
 struct TileDesc {
-    uint32_t task, rowBase, colBeg, seg;
+    uint32_t task, rowBase, colBeg;
 };
 
 // persistent top-2 matcher over a tile table split into kNumXcd lists

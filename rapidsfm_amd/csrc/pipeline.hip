@@ -139,7 +139,7 @@ Plan make_plan(const std::vector<rsfm_pipeline_pair>& pairs, uint32_t segCols, u
             if (t.nA == 0 || t.nB == 0) continue;
             for (uint32_t s = 0; s < t.nSeg; s++)
                 for (uint32_t r = 0; r < div_up(t.nA, bf::kBM); r++)
-                    pl.tiles.push_back(bf::TileDesc{(uint32_t)i, r * bf::kBM, s * segCols, s});
+                    pl.tiles.push_back(bf::TileDesc{(uint32_t)i, r * bf::kBM, s * segCols});
         }
     }
     pl.xcdOff[kNumXcd] = (uint32_t)pl.tiles.size();
