@@ -43,6 +43,26 @@
 #include <numeric>
 #include <vector>
 
+namespace rsfm_amd {
+namespace pipe {
+
+// Match results whose buffers are not 8-byte aligned: the matcher merges them by
+// 64-bit atomics in the arena, and they are copied out in words.
+struct CopyRange {
+    const uint32_t* src;
+    uint32_t* dst;
+    uint32_t words;
+};
+
+__global__ __launch_bounds__(256) void copy_kernel(const CopyRange* __restrict__ ranges)
+{
+    const CopyRange r = ranges[blockIdx.y];
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < r.words; i += gridDim.x * 256) r.dst[i] = r.src[i];
+}
+
+}  // namespace pipe
+}  // namespace rsfm_amd
+
 using namespace rsfm_amd;
 
 struct rsfm_pipeline {
@@ -66,6 +86,8 @@ struct rsfm_pipeline {
     uint32_t rmfCols = 0, rmfRows = 0;
     uint8_t* dPrep = nullptr;  // staging form of every pair's train descriptors
     uint32_t maxA = 0, maxB = 0;
+    pipe::CopyRange* dCopy = nullptr;  // misaligned result buffers
+    uint32_t nCopy = 0, maxCopy = 0;
     // chosen tiling
     uint32_t segCols = 0, wgPerXcd = 0, nTiles = 0, maxList = 0;
     float tunedMs = 0.f;
@@ -152,7 +174,7 @@ int upload(void* dst, const void* src, size_t bytes)
     return check_hip(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice), "pipeline upload");
 }
 
-// preparation + match of the current plan on stream s
+// preparation + match of the current plan on stream s, misaligned results copied out
 int enqueue_match(rsfm_pipeline* pl, hipStream_t s)
 {
     RSFM_CHECK(bf::launch_prep_table(pl->dTasks, (uint32_t)pl->pairs.size(), pl->maxA, pl->maxB, s));
@@ -161,6 +183,10 @@ int enqueue_match(rsfm_pipeline* pl, hipStream_t s)
             RSFM_CHECK(bf::launch_match_tile_grid_top2(pl->dTasks, pl->dTiles, pl->dXcdOff, pl->maxList, s));
         else
             RSFM_CHECK(bf::launch_match_tiles_top2(pl->dTasks, pl->dTiles, pl->dXcdOff, pl->wgPerXcd * kNumXcd, s));
+    }
+    if (pl->nCopy) {
+        pipe::copy_kernel<<<dim3(std::min<uint32_t>(div_up(pl->maxCopy, 256), 64), pl->nCopy), 256, 0, s>>>(pl->dCopy);
+        RSFM_CHECK(check_launch("pipeline result copy"));
     }
     return RSFM_OK;
 }
@@ -386,6 +412,22 @@ extern "C" int rsfm_pipeline_create(const rsfm_pipeline_pair* pairs, size_t nbPa
     const size_t oPoseF = take(P * sizeof(pose::DevTask));
     const size_t oPoseH = take(P * sizeof(pose::DevTask));
     const size_t oPrep = take(std::max<size_t>(1, worst.prepBytes));
+    // staging of result buffers that the matcher's 64-bit atomics cannot take
+    std::vector<pipe::CopyRange> copies;
+    std::vector<size_t> oCopies;
+    auto stage = [&](rsfm_best_match* p, uint32_t n) {
+        if (n == 0 || reinterpret_cast<uintptr_t>(p) % 8 == 0) return;
+        copies.push_back({nullptr, reinterpret_cast<uint32_t*>(p), 2 * n});
+        oCopies.push_back(take((size_t)n * sizeof(rsfm_best_match)));
+        pl->maxCopy = std::max(pl->maxCopy, 2 * n);
+    };
+    for (auto& x : pl->pairs) {
+        stage(x.bestA, x.nA);
+        stage(x.secondA, x.nA);
+        stage(x.bestB, x.nB);
+    }
+    pl->nCopy = (uint32_t)copies.size();
+    const size_t oCopy = take(std::max<size_t>(1, copies.size()) * sizeof(pipe::CopyRange));
     // 8-point solver: every hypothesis' model, so the best-model kernel reads
     // the winner instead of refitting it on one lane
     const size_t modelFloats = (size_t)cfg->nbHyp * 9;
@@ -410,6 +452,20 @@ extern "C" int rsfm_pipeline_create(const rsfm_pipeline_pair* pairs, size_t nbPa
     pl->dPoseF = reinterpret_cast<pose::DevTask*>(pl->arena + oPoseF);
     pl->dPoseH = reinterpret_cast<pose::DevTask*>(pl->arena + oPoseH);
     pl->dPrep = pl->arena + oPrep;
+    pl->dCopy = reinterpret_cast<pipe::CopyRange*>(pl->arena + oCopy);
+    // from here on the staged buffers stand in for the caller's
+    size_t next = 0;
+    auto staged = [&](rsfm_best_match*& p, uint32_t n) {
+        if (n == 0 || reinterpret_cast<uintptr_t>(p) % 8 == 0) return;
+        uint8_t* own = pl->arena + oCopies[next];
+        copies[next++].src = reinterpret_cast<uint32_t*>(own);
+        p = reinterpret_cast<rsfm_best_match*>(own);
+    };
+    for (auto& x : pl->pairs) {
+        staged(x.bestA, x.nA);
+        staged(x.secondA, x.nA);
+        staged(x.bestB, x.nB);
+    }
     float* dModels = reinterpret_cast<float*>(pl->arena + oModels);
     for (auto& x : pl->pairs) {
         pl->maxA = std::max(pl->maxA, x.nA);
@@ -493,7 +549,8 @@ extern "C" int rsfm_pipeline_create(const rsfm_pipeline_pair* pairs, size_t nbPa
         (rc = upload(pl->dDg, dg.data(), dg.size() * sizeof(degensac::DevTask))) != RSFM_OK ||
         (rc = upload(pl->dUnd, ud.data(), ud.size() * sizeof(undist::PairTask))) != RSFM_OK ||
         (rc = upload(pl->dPoseF, pf.data(), pf.size() * sizeof(pose::DevTask))) != RSFM_OK ||
-        (rc = upload(pl->dPoseH, ph.data(), ph.size() * sizeof(pose::DevTask))) != RSFM_OK)
+        (rc = upload(pl->dPoseH, ph.data(), ph.size() * sizeof(pose::DevTask))) != RSFM_OK ||
+        (rc = upload(pl->dCopy, copies.data(), copies.size() * sizeof(pipe::CopyRange))) != RSFM_OK)
         return fail_out(rc);
     pl->nUnd = (uint32_t)ud.size();
     pl->nPoseF = (uint32_t)pf.size();

@@ -173,6 +173,53 @@ def test_pipeline_pair_against_oracle(orc, dev):
     pl.close()
 
 
+# Match results of the first pairs at addresses that are multiples of 4 but not of 8, one
+# segment and several: the matcher's 64-bit atomics must not meet them, nothing past them changes
+@pytest.mark.parametrize("seg", [0, 1024])
+def test_pipeline_misaligned_results(dev, monkeypatch, seg):
+    from rapidsfm_amd import pipeline as P
+
+    _say("pipeline misaligned results", seg)
+    sizes = [(1000, 1200), (300, 9000), (400, 0), (0, 500), (2048, 2048), (1500, 8193)]
+    pairs = _batch(dev, sizes, seed=40)
+    bufs = {}
+    create = P.lib.rsfm_pipeline_create
+
+    class Lib:
+        def __getattr__(self, name):
+            return getattr(P_lib, name)
+
+        def rsfm_pipeline_create(self, arr, n, cfg, out):
+            a = ctypes.cast(arr, ctypes.POINTER(P.PipelinePair))
+            for i, (nA, nB) in enumerate(sizes[:-1]):
+                for field, m in (("bestA", nA), ("secondA", nA), ("bestB", nB)):
+                    t = torch.full((2 * m + 4,), -9, dtype=torch.int32, device=dev)
+                    assert t.data_ptr() % 8 == 0
+                    setattr(a[i], field, t.data_ptr() + 4)
+                    bufs[i, field] = t
+            torch.cuda.synchronize()
+            return create(arr, n, cfg, out)
+
+    P_lib = P.lib
+    monkeypatch.setattr(P, "lib", Lib())
+    pl = P.Pipeline(pairs, n_hyp=128, seed=500, seg_cols=seg)
+    ref = _reference(pairs, 128, 500)
+    for _ in range(2):
+        for t in bufs.values():
+            t.fill_(-9)
+        pl.run()
+        torch.cuda.synchronize()
+        for i, (nA, nB) in enumerate(sizes[:-1]):
+            for field, key, m in (("bestA", "bestA", nA), ("secondA", "secA", nA), ("bestB", "bestB", nB)):
+                t = bufs[i, field]
+                assert torch.equal(t[1:2 * m + 1].view(-1, 2), ref[i][key][:m]), (i, field)
+                assert int(t[0]) == -9 and bool((t[2 * m + 1:] == -9).all()), (i, field)
+                # what the common comparison looks at
+                pl.out[i][key][:m] = t[1:2 * m + 1].view(-1, 2)
+        _compare(pl, ref, pairs)
+    pl.close()
+
+
 CAM = (2000.0, 2000.0, 2000.0, 1500.0)
 
 
