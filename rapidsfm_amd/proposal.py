@@ -157,6 +157,7 @@ def subsample(rng, gt, outlier_rate):
 def score(problems, threshold=1.0):
     """problems: list of (pts (n,4), idx (H,8)) -> per-hypothesis counts and best masks; outputs
     share storage as ops.ransac_f8's do."""
+    problems = list(problems)
     likes = [pts for pts, _ in problems]
     counts = _rows(likes, [idx.shape[0] for _, idx in problems], None, torch.int32)
     masks = _rows(likes, [max(1, t.shape[0]) for t in likes], None, torch.uint8)

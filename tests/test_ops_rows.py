@@ -56,3 +56,17 @@ def test_current_stream_without_the_private_call(monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Stream)
     monkeypatch.setattr(ops, "_current_raw_stream", None, raising=False)
     assert ops._stream(None) == 42 and ops._stream(Stream) == 42
+
+
+def test_score_takes_any_iterable(monkeypatch):
+    from rapidsfm_amd import proposal
+
+    class Lib:
+        rsfm_ransac_f8 = staticmethod(lambda tasks, n, *a: 0 if n == 2 and tasks[1].nbPts == 30 else 1)
+
+    monkeypatch.setattr(proposal, "lib", Lib)
+    monkeypatch.setattr(proposal, "_stream", lambda s: 0)
+    pts = [torch.zeros(20, 4), torch.zeros(30, 4)]
+    idx = [torch.zeros((5, 8), dtype=torch.int32)] * 2
+    for outs in (proposal.score(list(zip(pts, idx))), proposal.score(zip(pts, idx))):
+        assert [len(o["mask"]) for o in outs] == [20, 30]
