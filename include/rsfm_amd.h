@@ -564,6 +564,8 @@ typedef struct rsfm_pipeline_pair {
     const void* descB;          /* device u8 [nB][128], 16-byte aligned */
     const float* kpA;           /* device (x, y) per query keypoint */
     const float* kpB;           /* device (x, y) per train keypoint */
+    /* match results, written in place when 8-byte aligned, else copied from memory of the
+     * pipeline's own */
     rsfm_best_match* bestA;     /* [nA] */
     rsfm_best_match* secondA;   /* [nA] */
     rsfm_best_match* bestB;     /* [nB] */

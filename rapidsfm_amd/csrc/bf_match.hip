@@ -673,10 +673,11 @@ struct Plan {
 // Columns per segment. Alone on its CU a workgroup takes about 6 us of its own
 // and 1 us per 64-column chunk (latency: the chip is far from full), so few row
 // blocks gain from short segments until every CU has a workgroup: one pair of
-// 1000 x 1187 took 23.0 us as four workgroups and takes 10.1 us as 36, 4096 x 4096 top-1 18.1 -> 11 us. Segments above 2048
-// columns are worth two workgroups per CU (16384 x 15411: 46.2 -> 44.8 us);
-// at 8192 x 8192 one and two per CU are equal (20.1, 20.7 us) and one merges
-// less.
+// 1000 x 1187 took 23.0 us as four workgroups and takes 10.2 us as 28 (seven
+// segments of 192 columns: the width is rounded up to whole chunks), 4096 x 4096
+// top-1 18.1 us as 64 and 10.0 as 256. Segments above 2048 columns are worth two
+// workgroups per CU (16384 x 15411: 46.2 -> 44.8 us); at 8192 x 8192 one and two
+// per CU are equal (20.1, 20.7 us) and one merges less.
 constexpr uint32_t kMinSegCols = 128;
 
 static Plan make_plan(const DevTask* t, size_t n, uint32_t maxSegCols)
@@ -882,8 +883,8 @@ extern "C" int rsfm_bf_match_top2(const rsfm_bf_top2_task* tasks, size_t nbTasks
 
 // ---------------------------------------------------------------------------
 // rsfm_bf_match_top2_noalloc: the top-2 matcher with its workspace (train
-// staging form) in a fixed device array instead of a
-// caller buffer, for callers that cannot allocate. The array is this file's
+// staging form) in a fixed device array instead of a caller buffer, for callers
+// that cannot allocate. The array is this file's
 // `scratch`; its device address is looked up once per device, with that device
 // current, and only that address is handed to kernels. Every call on one GPU
 // shares the array (calls that overlap on one GPU race); nothing in it needs

@@ -9,10 +9,10 @@
 // random_device-seeded engine), so a fixed index set gives one defined
 // inlier count per hypothesis.
 //
-// GPU layout: a workgroup of four wavefronts fits its hypotheses one per lane
-// (fgeom::fit8) into LDS, then counts their inliers over all correspondences
-// with the matrix-core screen of screen.hpp (fundamental matrices) or one lane
-// per hypothesis (homographies).
+// GPU layout: a workgroup of four or eight wavefronts fits its hypotheses one
+// per lane (fgeom::fit8) into LDS, then counts their inliers over all
+// correspondences with the matrix-core screen of screen.hpp (fundamental
+// matrices) or one lane per hypothesis (homographies, four wavefronts).
 #include "internal.hpp"
 #include "fgeom.hpp"
 #include "hgeom.hpp"
@@ -218,7 +218,8 @@ __device__ inline screen::Box box_join(const Sm& S, uint32_t first, uint32_t n)
     return screen::box_finish(b, n);
 }
 
-// Scoring of fundamental matrices: a workgroup of eight wavefronts holds 64 kFit
+// Scoring of fundamental matrices: a workgroup of kWaves wavefronts (eight in
+// the wide form, four in the narrow one, see launch_score) holds 64 kFit
 // hypotheses, fitted one per lane by its first kFit wavefronts while the others
 // scan the pair's box; then the wavefronts count the inliers of 16 kNB
 // hypotheses each, kSplit of them sharing the points, with the matrix-core
@@ -893,7 +894,7 @@ int launch_sample_table(const SampleTask* tasks, uint32_t nTasks, uint32_t maxH,
 // pairs x 4096 hypotheses x 1300-2400 points (192 or 768 workgroups) the wide
 // form takes 53 us and the narrow one 58 us, at one pair (16 or 64) only the
 // narrow one spreads the fits. 32 pairs x 4096 x 2454 points: 208 -> 98 us
-// against one exact test per lane and trip (VALU issue 84% busy; 46.6 M vector
+// against one exact test per lane and trip (VALU issue 93% busy; 46.6 M vector
 // instructions instead of 110 M), 64 pairs of the affine-filtered batch 218 ->
 // 139 us.
 constexpr uint32_t kWideMin = 128;

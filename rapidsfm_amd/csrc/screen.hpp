@@ -37,8 +37,10 @@
 // With d and c the sums of these for e and for D (d^2 and the comparison's own
 // roundings in c), the exact e^2 - D differs from the screen's by at most
 // 2 d |e| + c where it is near zero, so a test with g > c has the exact
-// outcome. The others are open (4e-5 of the tests on 70% outliers, 6e-3 on 5%)
-// and are done by the exact test in groups of the lane's four.
+// outcome. The others are open and are done by the exact test in groups of the
+// lane's four: 2e-4 to 3e-4 of all tests are in such a group at 70% outliers,
+// 2e-3 to 3e-3 at 30%, 1e-2 to 2e-2 at 5% (600 and 2454 points, 8 points a model;
+// 7-point models up to 1.3e-3 at 70%).
 #pragma once
 #include "common.hpp"
 #include "fgeom.hpp"
